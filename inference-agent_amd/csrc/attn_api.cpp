@@ -126,12 +126,12 @@ size_t ingot_linear_weight_bytes(const IngotLinearDesc* d) {
 
 uint32_t ingot_linear_splits(const IngotLinearDesc* d) {
     if (check_linear(d)) return 0;
-    return ingot::linear_splits(d->n_in, d->n_out, d->n_tok, d->n_splits, ~size_t(0));
+    return ingot::linear_splits(d->type, d->n_in, d->n_out, d->n_tok, d->n_splits, ~size_t(0));
 }
 
 size_t ingot_linear_workspace_size(const IngotLinearDesc* d) {
     if (check_linear(d)) return 0;
-    return ingot::linear_workspace_size(d->n_in, d->n_out, d->n_tok, d->n_splits);
+    return ingot::linear_workspace_size(d->type, d->n_in, d->n_out, d->n_tok, d->n_splits);
 }
 
 int ingot_linear(const void* w, const float* x, float* out, void* workspace, size_t workspace_bytes,

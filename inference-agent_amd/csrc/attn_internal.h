@@ -107,9 +107,10 @@ int launch_proj(uint32_t type, const void* const* W, const float* x, const float
                 int pro, int epi, float eps, hipStream_t stream, const ProjRope* rope = nullptr,
                 uint32_t n_tok = 1);
 // Split count for the batched path (requested: 0 = choose); `workspace_bytes` bounds it.
-uint32_t linear_splits(uint32_t n_in, uint32_t n_out, uint32_t n_tok, uint32_t requested,
+uint32_t linear_splits(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_tok, uint32_t requested,
                        size_t workspace_bytes);
-size_t linear_workspace_size(uint32_t n_in, uint32_t n_out, uint32_t n_tok, uint32_t requested);
+size_t linear_workspace_size(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_tok,
+                             uint32_t requested);
 
 // Per-layer model ops (model_ops.hip). Return 0, -1 (grid too large) or -4 (launch failed).
 int launch_rmsnorm(const float* x, const float* w, float* out, uint32_t n, uint32_t n_rows, float eps,

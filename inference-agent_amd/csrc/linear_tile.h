@@ -1,0 +1,51 @@
+// linear_tile.h — the launcher of the batched linear kernel (linear_tile.hip), one object per
+// weight type.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace ingot {
+
+// Shape of a call's workgroups: NTB token blocks of 32 per tile (1..5), KG k groups among the
+// eight waves (1, 2 or 4: a tile has 256 / KG rows), and the ways n_in is split over workgroups.
+struct TileShape {
+    uint32_t ntb, kg, splits;
+};
+
+struct TileCall {
+    const uint8_t* W[3];
+    float* out[3];
+    uint32_t n_out[3];
+    uint32_t n_mats;
+    const float* x;
+    uint32_t n_in, n_tok;
+    bool accumulate;
+    bool pair;  // W = (gate, up): out[0] = silu(gate) * up
+    TileShape shape;
+    void* workspace;  // counters, then partial tiles (shape.splits > 1)
+    hipStream_t stream;
+};
+
+// Rows per tile, k elements per stage and bytes of one partial tile of a shape.
+constexpr uint32_t tile_rows(uint32_t kg) { return 256 / kg; }
+// A stage: 64-element steps of each k group (two where one k group fits the LDS), and elements.
+constexpr uint32_t tile_cols(uint32_t kg) { return kg == 1 ? 2 : 1; }
+constexpr uint32_t tile_stage(uint32_t kg) { return 64 * kg * tile_cols(kg); }
+// A k group's share of n_in is a multiple of this many elements (whole Q6_K blocks).
+constexpr uint32_t tile_unit(int type) { return type == 14 ? 256 : 64; }
+// The two x buffers.
+constexpr size_t tile_x_lds(uint32_t ntb, uint32_t kg) { return size_t(2) * 32 * ntb * tile_stage(kg) * 2; }
+// LDS of a workgroup: the x buffers and the waves' weights, reused by the reduction over the k
+// groups and the silu exchange (16 floats per lane, token block and wave).
+constexpr size_t tile_lds(uint32_t ntb, uint32_t kg, size_t w) {
+    const size_t x = tile_x_lds(ntb, kg) + w;
+    const size_t red = size_t(kg - 1) * (8 / kg) * ntb * 4096, silu = size_t(4 / kg) * ntb * 4096;
+    return x > red ? (x > silu ? x : silu) : (red > silu ? red : silu);
+}
+constexpr size_t tile_bytes(const TileShape& s) { return size_t(tile_rows(s.kg)) * s.ntb * 32 * 4; }
+
+// 0, -1 (grid too large or a bad shape) or -4 (launch failed). T: the GGUF type id.
+template <int T> int launch_tile(const TileCall& c);
+
+}  // namespace ingot

@@ -1,0 +1,69 @@
+"""The batched linear kernel at the edges of its tiles: token blocks of 32 (and where the number of
+k groups changes), tiles of 64 / 128 / 256 rows, k shares that end inside a step of 64 elements,
+against the CPU oracle with both operands rounded to f16. The bar is the one of test_gpu_linear:
+only the order of the f32 sums differs (rel-L2 <= 1e-5, max|d| <= 1e-5 * max|ref| + 1e-6)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import ensure_built
+
+import gguf_blocks as gb
+
+pytestmark = pytest.mark.gpu
+
+TYPES = ["F32", "F16", "BF16", "Q8_0", "Q4_0", "Q4_1", "Q6_K"]
+
+
+@pytest.fixture(scope="module")
+def dev():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.fail("GPU test run without a GPU")
+    ensure_built("lib")
+    import ingot_attn
+
+    ingot_attn.load_library()
+    return torch.device("cuda:0")
+
+
+def _run(dev, t, raw, x, n_in, n_out, n_splits):
+    import torch
+    import ingot_attn as ia
+
+    out = torch.full((x.shape[0] * n_out + 64,), float("nan"), device=dev)
+    ia.linear(torch.from_numpy(raw.reshape(-1)).to(dev), torch.from_numpy(x).to(dev), out,
+              ia.linear_desc(t, n_in, n_out, x.shape[0], n_splits=n_splits), workspace=ia.Workspace(dev))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.all(np.isnan(got[x.shape[0] * n_out:])), "wrote past its rows"
+    return got[: x.shape[0] * n_out].reshape(x.shape[0], n_out)
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("n_tok,n_in,n_out,n_splits", [
+    (2, 32, 1, 0), (31, 96, 33, 0), (33, 160, 65, 1), (64, 288, 63, 0), (96, 352, 129, 1), (97, 1056, 130, 0),
+    (129, 2336, 127, 3), (288, 544, 257, 1), (289, 1312, 255, 1), (300, 800, 31, 2)])
+def test_tile_edges(dev, oracle_mod, t, n_tok, n_in, n_out, n_splits):
+    n_in = n_in if t != "Q6_K" else -(-n_in // 256) * 256
+    raw = gb.random_weights(t, n_out, n_in, seed=n_tok + n_in)
+    x = np.random.default_rng(n_out).standard_normal((n_tok, n_in)).astype(np.float32)
+    got = _run(dev, t, raw, x, n_in, n_out, n_splits)
+    want = oracle_mod.linear(t, raw, x, n_in, n_out, f16_path=True)
+    d = np.abs(got - want)
+    assert np.all(np.isfinite(got))
+    assert d.max() <= 1e-5 * np.abs(want).max() + 1e-6 and np.linalg.norm(d) <= 1e-5 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("t", ["F16", "Q8_0"])
+def test_ragged_end_reads_no_neighbour(dev, t):
+    """A row whose share of n_in ends inside a step: the elements past its end are the next row's
+    and must not reach the sum, not even where that row is infinite."""
+    n_in, n_out, n_tok = 96, 6, 5
+    raw = gb.random_weights(t, n_out, n_in, seed=3).copy()
+    raw.view(np.uint8).reshape(n_out, -1)[4, 0:2] = (0x00, 0x7C)  # an infinite value or scale
+    x = np.random.default_rng(4).standard_normal((n_tok, n_in)).astype(np.float32)
+    got = _run(dev, t, raw, x, n_in, n_out, 0)
+    assert np.all(np.isfinite(np.delete(got, 4, axis=1))) and not np.any(np.isfinite(got[:, 4]))
