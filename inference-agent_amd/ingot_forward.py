@@ -22,29 +22,28 @@ import ingot_attn as ia
 
 
 # Tiles (256 rows x 64 tokens over q, k and v) from which a chunk's q/k/v run as one batched
-# launch; a test sets 0 to force that path.
-QKV_ONE_LAUNCH_MIN_TILES = 128
+# launch: every chunk (Llama-3.2-3B Q4_0: 13 tokens 12.9 us in one launch, 25 in three; 157 tokens
+# 24.1 and 33.8; 512 tokens 34.8 and 56.7). A number above a chunk's tiles forces the three launches.
+QKV_ONE_LAUNCH_MIN_TILES = 0
 
 
 def qkv_one_launch(n_tok, q_dim, kv_dim):
     """Whether a chunk's q/k/v run as one batched launch (ingot_proj, no split-K) rather than
-    three ingot_linear calls (each split-K over the 256 CUs): when the three matrices' tiles of
-    256 rows x 64 tokens reach half the CUs together (Llama-3.2-3B at 512 tokens: 160 tiles; at
-    256 tokens 80, where three split launches are faster)."""
+    three ingot_linear calls (each split-K over the 256 CUs)."""
     rows = -(-q_dim // 256) + 2 * -(-kv_dim // 256)
     return rows * -(-n_tok // 64) >= QKV_ONE_LAUNCH_MIN_TILES
 
 
 # Tiles (128 rows of gate and of up x 64 tokens) from which a chunk's gate/up + silu run as one
-# batched launch; a test sets 0 to force that path.
-FFN_ONE_LAUNCH_MIN_TILES = 256
+# batched launch: every chunk (Llama-3.2-3B Q4_0: 13 tokens 18.1 us in one launch, 25.1 in two before
+# ingot_silu_mul; 157 tokens 36.7 and 49.3).
+FFN_ONE_LAUNCH_MIN_TILES = 0
 
 
 def ffn_one_launch(n_tok, n_ff):
     """Whether a chunk's gate and up projections and silu(gate) * up run as one batched launch
-    (ingot_proj with the silu epilogue, no split-K) rather than two ingot_linear calls (each
-    split-K over the CUs when its tiles are few) and ingot_silu_mul: once the paired tiles fill
-    the 256 CUs (Llama-3.2-3B: 512 tiles at 512 tokens, 256 at 256)."""
+    (ingot_proj with the silu epilogue, no split-K) rather than two ingot_linear calls and
+    ingot_silu_mul."""
     return -(-n_ff // 128) * -(-n_tok // 64) >= FFN_ONE_LAUNCH_MIN_TILES
 
 
