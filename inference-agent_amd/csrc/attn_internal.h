@@ -59,6 +59,13 @@ int launch_prefill(const float* q, const _Float16* k, const _Float16* v, float* 
                    uint32_t group, uint32_t head_dim, uint32_t n_splits, float scale,
                    hipStream_t stream);
 
+// Prefill at a head size below 256 that is a multiple of 8 and none of those three, on the same
+// kernel with f32 accuracy (two f16 parts of q and of the probabilities); never split, no records.
+// -2 for other head sizes.
+int launch_prefill_exact(const float* q, const _Float16* k, const _Float16* v, float* out, uint32_t pos,
+                         uint32_t n_tok, uint32_t q_stride, uint32_t n_head_kv, uint32_t group,
+                         uint32_t head_dim, float scale, hipStream_t stream);
+
 // Attention for head sizes without an MFMA kernel (attn_naive.hip): head_dim 1..1024, decode
 // (pos = n_keys - 1, n_tok = 1) and causal prefill. Decode splits the keys into
 // attn_any_slices(n_keys, 1) slices whose records (head_dim + 2 floats each, per head) go to

@@ -87,12 +87,24 @@ template <int HD> __device__ __forceinline__ int swz_v(int row) {
     return HD == 64 ? ((row >> 1) & 3) << 1 : (row & 7) << 1;
 }
 
-template <int HD, int G, int QW, int KG>
+// EXACT: head sizes without a kernel of their own (hd < HD, a multiple of 8), one head per unit,
+// never split: the dims past hd are zero in LDS and not stored, and q and the probabilities enter
+// the MFMAs as two f16 parts each (hi + lo, together ~22 bits; K and V are f16 as stored), so that
+// the scores and the sums keep the f32 accuracy of the fallback kernel at twice the matrix work.
+// A query row is first scaled by a power of two that puts its largest element at 2^8..2^9 (any
+// finite q then fits the f16 parts, and a small one keeps its low bits); the scores are scaled
+// back in f32. Bound by the LDS reads and the chain of the longest key walk, like a short chunk of
+// a 128-wide head: 24 / 8 heads of 96, 301 tokens at 211, 82 -> 13 us (154 TFLOP/s of useful
+// products), error against 64 bits 3.6e-7 -> 2.4e-7.
+template <int HD, int G, int QW, int KG, bool EXACT = false>
 __global__ __launch_bounds__(64 * QW * KG) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict__ K,
                          const _Float16* __restrict__ V, float* __restrict__ out,
                          char* __restrict__ part, uint32_t pos, uint32_t n_tok, uint32_t q_stride,
-                         uint32_t n_head_kv, uint32_t kv_div, uint32_t tps, float qscale) {
+                         uint32_t n_head_kv, uint32_t kv_div, uint32_t tps, float qscale, uint32_t hd_) {
+    static_assert(!EXACT || G == 1, "one head per unit");
+    const uint32_t hd = EXACT ? hd_ : HD;
+    constexpr int GQ = EXACT ? 2 : G;  // f16 rows of q per query: the unit's heads, or hi and lo
     constexpr int BN = kBN<HD>, RB = kRowBytes<HD>, CPR = kChunks<HD>, TB = kTileBytes<HD>, SB = kStageBytes<HD>;
     constexpr int HALVES = BN / 32;  // 32-key halves per tile
     constexpr int PB = HD * 2 + 16;  // bytes per split record: o[HD] / l as f16, then {m, l, 0, 0}
@@ -127,7 +139,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
     // (n_head_kv counts units, kv_div of them per KV head): the group's heads run in separate
     // workgroups, each reading the same K/V.
     const uint32_t kvh = blockIdx.x % n_head_kv;
-    const size_t kv_dim = size_t(n_head_kv / kv_div) * HD;
+    const size_t kv_dim = size_t(n_head_kv / kv_div) * hd;
     uint32_t qblk = (n_tok + 16 * QW - 1) / (16 * QW), split = blockIdx.x / n_head_kv, n_splits = 1;
     uint32_t ntiles = 0;
     while (qblk > 0) {
@@ -150,8 +162,8 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
     const uint32_t kend_w = q0 < n_tok ? pos + min(n_tok, q0 + 16) : 0;
     const uint32_t qpos = pos + q0 + li;  // this lane's query position
 
-    const _Float16* Kg = K + size_t(kvh / kv_div) * HD;
-    const _Float16* Vg = V + size_t(kvh / kv_div) * HD;
+    const _Float16* Kg = K + size_t(kvh / kv_div) * hd;
+    const _Float16* Vg = V + size_t(kvh / kv_div) * hd;
 
     // Tile copy HBM -> LDS: 2*NIT buffer_load ... lds instructions of 1 KB (RPI rows) per tile
     // (HD 128: 32 of 4 rows), spread over the waves of the key group and issued in two groups
@@ -172,6 +184,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
         const int row = RPI * (i % NIT) + lane / CPR;
         const int logical = (lane % CPR) ^ (isv ? swz_v<HD>(row) : swz_k<HD>(row));
         dma_off[k] = uint32_t(row) * row_bytes + 16u * uint32_t(logical);
+        if (EXACT && 8u * uint32_t(logical) >= hd) dma_off[k] = 0x80000000u;  // past the range: zeros
     }
     // Copy instruction k (0 .. kInstPerWave-1) of this wave for tile t into buffer `buf`.
     auto issue_inst = [&](uint32_t t, int buf, int k) {
@@ -193,23 +206,25 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
     // at c ^ (query % CPR), so that the B-operand reads below are (nearly) bank-conflict free.
     // All of the thread's Q loads are issued first, then the first tile's copy: loads complete
     // in order, so the conversion waits only for Q, and the tile streams in meanwhile.
-    static_assert(QW * 16 == 64 && G * 32 * RB <= SB, "Q staging fits the free stages");
+    static_assert(QW * 16 == 64 && GQ * 32 * RB <= SB, "Q staging fits the free stages");
     constexpr int QF4 = HD / 4;            // float4 chunks of one (query, head) row
     constexpr int kF4 = QW * 16 * G * QF4;  // float4 chunks of the workgroup's Q
     constexpr int NT = 64 * QW * KG;
     constexpr int kQIt = (kF4 + NT - 1) / NT;
     float4v qx[kQIt];
+    __shared__ float qback[EXACT ? QW * 16 : 1];  // per query: the power of two that scales its scores back
     {
         const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(q + size_t(qblk0) * q_stride + size_t(kvh) * G * HD), 0,
+            const_cast<float*>(q + size_t(qblk0) * q_stride + size_t(kvh) * G * hd), 0,
             0x7fffffff, kBufferFlags);
 #pragma unroll
         for (int it = 0; it < kQIt; it++) {
             const int idx = min(tid + it * NT, kF4 - 1);
             const int ql = idx / (G * QF4), rem = idx % (G * QF4);
             const uint32_t row = min(qblk0 + ql, n_tok - 1) - qblk0;
+            const bool past = EXACT && 4 * uint32_t(rem) >= hd;
             qx[it] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(
-                qr, int(4 * (row * q_stride + (rem / QF4) * HD + 4 * (rem % QF4))), 0, 0));
+                qr, past ? int(0x80000000u) : int(4 * (row * q_stride + (rem / QF4) * HD + 4 * (rem % QF4))), 0, 0));
         }
     }
     uint32_t t_first = t_begin + kg;
@@ -222,21 +237,39 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
         if (kF4 % NT != 0 && idx >= kF4) break;
         const int ql = idx / (G * QF4), rem = idx % (G * QF4);
         const int h = rem / QF4, c4 = rem % QF4;
-        half4 y;
+        half4 y, lo;
+        float unit = qscale;
+        if constexpr (EXACT) {
+            // the row's largest element, over its QF4 consecutive lanes
+            float x = fmaxf(fmaxf(fabsf(qx[it][0]), fabsf(qx[it][1])), fmaxf(fabsf(qx[it][2]), fabsf(qx[it][3])));
 #pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = _Float16(qx[it][e] * qscale);
+            for (int o = 1; o < QF4; o <<= 1) x = fmaxf(x, __shfl_xor(x, o));
+            const int e = 8 - min(max(int(__float_as_uint(x * qscale) >> 23) - 127, -100), 100);
+            unit = 1.f;
+            qx[it] = qx[it] * qscale * ldexpf(1.f, e);
+            if (c4 == 0) qback[ql] = ldexpf(1.f, -e);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float f = qx[it][e] * unit;
+            y[e] = _Float16(f);
+            lo[e] = _Float16(f - float(y[e]));
+        }
         char* qs = stage_of(ql >> 5, 1);
         const int chunk = (c4 >> 1) ^ (ql % CPR);
-        *reinterpret_cast<half4*>(qs + ((ql & 31) * G + h) * RB + 16 * chunk + 8 * (c4 & 1)) = y;
+        char* dst = qs + ((ql & 31) * GQ + h) * RB + 16 * chunk + 8 * (c4 & 1);
+        *reinterpret_cast<half4*>(dst) = y;
+        if constexpr (EXACT) *reinterpret_cast<half4*>(dst + RB) = lo;
     }
     __syncthreads();
     // B operand Q^T per head: lane holds Q[q0 + li][32*ks + 8*g + e] * scale*log2(e), as f16.
-    half8 qb[G][KS];
+    half8 qb[GQ][KS];
+    const float back = EXACT ? qback[EXACT ? 16 * qw + li : 0] : 1.f;
     {
         const int ql = 16 * qw + li;
-        const char* qs = stage_of(ql >> 5, 1) + (ql & 31) * G * RB;
+        const char* qs = stage_of(ql >> 5, 1) + (ql & 31) * GQ * RB;
 #pragma unroll
-        for (int h = 0; h < G; h++)
+        for (int h = 0; h < GQ; h++)
 #pragma unroll
             for (int ks = 0; ks < KS; ks++)
                 qb[h][ks] = *reinterpret_cast<const lds_half8*>(
@@ -278,7 +311,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
         // Halves of 32 keys (scores, online-softmax update, P*V each), so only 32 keys' worth
         // of S and P is live at a time.
         float4v S[2][G];
-        half8 P[G];
+        half8 P[GQ];
         auto scores = [&](int hs) {
 #pragma unroll
             for (int T = 0; T < 2; T++) {
@@ -289,8 +322,13 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
                     const half8 a = *reinterpret_cast<const lds_half8*>((const lds_void*)(Ks + row * RB + 16 * chunk));
 #pragma unroll
                     for (int h = 0; h < G; h++)
-                        S[T][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[h][ks], ks == 0 ? negm[h] : S[T][h], 0, 0, 0);
+                        S[T][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[h][ks], ks == 0 ? (EXACT ? float4v{0.f, 0.f, 0.f, 0.f} : negm[h]) : S[T][h], 0, 0, 0);
+                    if constexpr (EXACT)
+                        S[T][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[1][ks], S[T][0], 0, 0, 0);
                 }
+                if constexpr (EXACT)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) S[T][0][j] = fmaf(S[T][0][j], back, negm[0][j]);
             }
         };
         auto softmax = [&](int hs) {
@@ -331,7 +369,8 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
                     x = max_lanes4(x);  // max over the 4 lanes of a query
                     const bool grow = started[h] ? (x > kLazy) : (x > -__builtin_inff());
                     const float delta = grow ? x : 0.f;
-                    const float alpha = fast_exp2(-delta);
+                    // (a first maximum may be far below 0: nothing is accumulated yet to rescale)
+                    const float alpha = started[h] ? fast_exp2(-delta) : 0.f;
                     m[h] += delta;
                     negm[h] = float4v{-m[h], -m[h], -m[h], -m[h]};
                     l[h] *= alpha;
@@ -351,7 +390,19 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
 #pragma unroll
                 for (int T = 0; T < 2; T++)
 #pragma unroll
-                    for (int j = 0; j < 4; j++) P[h][4 * T + j] = _Float16(fast_exp2(S[T][h][j]));
+                    for (int j = 0; j < 4; j++) {
+                        const float p = fast_exp2(S[T][h][j]);
+                        P[h][4 * T + j] = _Float16(p);
+                        if constexpr (EXACT) {
+                            P[1][4 * T + j] = _Float16(p - float(P[0][4 * T + j]));
+                            S[T][0][j] = p;
+                        }
+                    }
+                if constexpr (EXACT) {  // (the eight summed first: a shorter chain of roundings)
+                    l[0] += ((S[0][0][0] + S[0][0][1]) + (S[0][0][2] + S[0][0][3])) +
+                            ((S[1][0][0] + S[1][0][1]) + (S[1][0][2] + S[1][0][3]));
+                    break;
+                }
                 const half2v one = {_Float16(1.f), _Float16(1.f)};
                 float ls = l[h];
 #pragma unroll
@@ -360,7 +411,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
                 l[h] = ls;
             }
         };
-        auto pv = [&](int hs, const half8 (&Pp)[G]) {
+        auto pv = [&](int hs, const half8 (&Pp)[GQ]) {
             // O^T (128 dims x (G x 16 queries)) += V^T (128 x 32) P^T (32 x 16) per head.
 #pragma unroll
             for (int d = 0; d < ND; d++) {
@@ -376,6 +427,11 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
                     part_[half_] = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4f16(src));
                 }
                 const half8 a = __builtin_shufflevector(part_[0], part_[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                if constexpr (EXACT) {  // (32 keys summed on their own, then one rounding into O)
+                    float4v t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, Pp[1], float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    O[0][d] += __builtin_amdgcn_mfma_f32_16x16x32_f16(a, Pp[0], t, 0, 0, 0);
+                    continue;
+                }
 #pragma unroll
                 for (int h = 0; h < G; h++)
                     O[h][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, Pp[h], O[h][d], 0, 0, 0);
@@ -528,11 +584,12 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
         for (int h = 0; h < G; h++) {
             const uint32_t head = kvh * G + h;
             const float inv = l[h] > 0.f ? 1.f / l[h] : 0.f;
-            const int off = int(4 * ((row - qblk0) * q_stride + head * HD + 4 * g));
+            const int off = int(4 * ((row - qblk0) * q_stride + head * hd + 4 * g));
 #pragma unroll
             for (int d = 0; d < ND; d++)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, O[h][d] * inv), ors, off + 64 * d, 0,
-                                                       kScDevice);
+                if (!EXACT || uint32_t(16 * d + 4 * g) < hd)
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, O[h][d] * inv), ors, off + 64 * d,
+                                                           0, kScDevice);
         }
         return;
     }
@@ -633,7 +690,7 @@ int launch_prefill_g(const float* q, const _Float16* k, const _Float16* v, float
     if (uint64_t(pairs) * n_head_kv > 0x7fffffffu) return -1;
     const dim3 grid(pairs * n_head_kv);
     hipLaunchKernelGGL((attn_prefill_kernel<HD, G, kQW, kKG>), grid, dim3(64 * kQW * kKG), 0, stream,
-                       q, k, v, out, part, pos, n_tok, q_stride, n_head_kv, kv_div, tps, qscale);
+                       q, k, v, out, part, pos, n_tok, q_stride, n_head_kv, kv_div, tps, qscale, uint32_t(HD));
     if (hipGetLastError() != hipSuccess) return -4;
     if (n_splits > 1) {
         const uint32_t n_head = n_head_kv * G;
@@ -727,6 +784,31 @@ int launch_prefill_hd(const float* q, const _Float16* k, const _Float16* v, floa
 }
 
 }  // namespace
+
+namespace {
+
+template <int HD>
+int launch_exact_hd(const float* q, const _Float16* k, const _Float16* v, float* out, uint32_t pos,
+                    uint32_t n_tok, uint32_t q_stride, uint32_t n_head_kv, uint32_t group, uint32_t head_dim,
+                    float scale, hipStream_t stream) {
+    const uint64_t wgs = uint64_t((n_tok + kQBlock - 1) / kQBlock) * n_head_kv * group;
+    if (wgs > 0x7fffffffu) return -1;
+    hipLaunchKernelGGL((attn_prefill_kernel<HD, 1, kQW, kKG, true>), dim3(uint32_t(wgs)), dim3(64 * kQW * kKG), 0,
+                       stream, q, k, v, out, nullptr, pos, n_tok, q_stride, n_head_kv * group, group,
+                       (pos + n_tok + kBN<HD> - 1) / kBN<HD>, scale * kLog2e, head_dim);
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+}  // namespace
+
+int launch_prefill_exact(const float* q, const _Float16* k, const _Float16* v, float* out, uint32_t pos,
+                         uint32_t n_tok, uint32_t q_stride, uint32_t n_head_kv, uint32_t group,
+                         uint32_t head_dim, float scale, hipStream_t stream) {
+    if (head_dim % 8 != 0 || head_dim > 256) return -2;
+    if (head_dim < 64) return launch_exact_hd<64>(q, k, v, out, pos, n_tok, q_stride, n_head_kv, group, head_dim, scale, stream);
+    if (head_dim < 128) return launch_exact_hd<128>(q, k, v, out, pos, n_tok, q_stride, n_head_kv, group, head_dim, scale, stream);
+    return launch_exact_hd<256>(q, k, v, out, pos, n_tok, q_stride, n_head_kv, group, head_dim, scale, stream);
+}
 
 int launch_prefill(const float* q, const _Float16* k, const _Float16* v, float* out, char* part,
                    uint32_t pos, uint32_t n_tok, uint32_t q_stride, uint32_t n_head_kv,

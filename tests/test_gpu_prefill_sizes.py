@@ -1,0 +1,58 @@
+"""Prefill at head sizes that share the MFMA kernel with zero-filled dims (multiples of 8 below 256
+other than 64 and 128): against a float64 reference on the CPU. q and the probabilities enter as
+two f16 parts (a relative 2^-22 each), sums are f32: with scores of magnitude s the result is off by
+about (s + 4) * 2^-22, so rel-L2 <= 2e-6 at s ~ 4 and <= 2e-5 at s ~ 100 (the first maximum of a
+key group may then lie far below zero)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import ensure_built
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.fail("GPU test run without a GPU")
+    ensure_built("lib")
+    import ingot_attn
+
+    ingot_attn.load_library()
+    return torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("hd,nh,nkv,pos,n,pad", [
+    (8, 2, 1, 0, 2, 0), (56, 4, 2, 31, 33, 0), (72, 3, 1, 63, 65, 3), (96, 6, 2, 127, 64, 0),
+    (120, 2, 2, 190, 129, 1), (136, 4, 1, 5, 70, 0), (248, 2, 1, 33, 31, 2)])
+@pytest.mark.parametrize("gain,bar", [(1.0, 2e-6), (100.0, 2e-5)])
+def test_zero_filled_dims(dev, hd, nh, nkv, pos, n, pad, gain, bar):
+    import torch
+    import ingot_attn as ia
+
+    rng = np.random.default_rng(hd + n)
+    L, kvd, stride = pos + n, nkv * hd, nh * hd + pad
+    q = (rng.standard_normal((n, stride)) * gain).astype(np.float32)
+    # a layer behind a slice of NaNs: nothing outside the visible rows may be read into a sum
+    k = np.full((2 * L, kvd), np.nan, np.float16)
+    v = np.full((2 * L, kvd), np.nan, np.float16)
+    k[L:] = rng.standard_normal((L, kvd)).astype(np.float16)
+    v[L:] = rng.standard_normal((L, kvd)).astype(np.float16)
+    t = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+    out = torch.full((n, stride), float("nan"), device=dev)
+    ia.attn_prefill(t(q), t(k), t(v), out, ia.prefill_desc(nh, nkv, hd, pos, n, kv_offset=L * kvd, q_stride=stride))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.all(np.isnan(got[:, nh * hd:])), "wrote past the heads"
+    for h in range(nh):
+        c = slice((h // (nh // nkv)) * hd, (h // (nh // nkv) + 1) * hd)
+        s = q[:, h * hd:(h + 1) * hd].astype(np.float64) @ k[L:, c].astype(np.float64).T / np.sqrt(hd)
+        s[np.arange(L)[None, :] > pos + np.arange(n)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        want = p / p.sum(1, keepdims=True) @ v[L:, c].astype(np.float64)
+        d = got[:, h * hd:(h + 1) * hd] - want
+        assert np.all(np.isfinite(d)) and np.linalg.norm(d) <= bar * np.linalg.norm(want), f"head {h}"
