@@ -845,15 +845,18 @@ uint64_t tile_count(uint32_t n_out, uint32_t n_tok, const TileShape& s) {
     return uint64_t((n_out + tr - 1) / tr) * ((nb + s.ntb - 1) / s.ntb);
 }
 
-// A call that is not split: the number of k groups depends on n_tok only, so that every output is
-// summed in the same order whatever else shares the launch (ingot_proj equals ingot_linear bit for
-// bit); the tile height, which does not change the order, is the one that takes least time for
-// n_out rows. Four k groups up to 96 tokens (13 tokens, q/k/v of 3072 x 5120 Q4_0: 12.9 us
-// against 23.6 with two; gate/up 18.0 against 30.0), two up to 288 (gate/up at 157 tokens: 37.1
-// against 49.5 with four, 38.9 with one), then one (gate/up at 512 tokens: 67 against 88).
-TileShape unsplit_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_tok) {
+// A call that is not split: the number of k groups depends on n_tok and on which side of 4096 rows
+// each matrix is, so that every output is summed in the same order whatever else shares the launch
+// (ingot_proj equals ingot_linear bit for bit; it launches matrices of both sides apart). The tile
+// height, which does not change the order, is the one that takes least time for n_out rows.
+// Measured on Q4_0 rows of 3072 (four, two, one k groups, us): gate/up of 2 x 8192 rows at 70
+// tokens 27.7 / 31 / 38, at 157 49.5 / 37.1 / 38.9, at 512 143 / 88 / 67; q/k/v of 3072 + 2 x 1024
+// rows at 157 tokens 17.4 / 24.3 / 33.7, at 256 23.2 / 26.2 / 34.7, at 389 41.4 / 29.8 / 34.7, at
+// 512 44 / 32.8 / 35.2.
+constexpr uint32_t kNarrowRows = 4096;
+TileShape unsplit_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_tok, bool narrow) {
     const uint32_t nb = (n_tok + 31) / 32;
-    TileShape best{0, nb <= 3 ? 4u : nb <= 9 ? 2u : 1u, 1};
+    TileShape best{0, narrow ? (nb <= 9 ? 4u : 2u) : nb <= 3 ? 4u : nb <= 9 ? 2u : 1u, 1};
     float t = 0;
     for (uint32_t ntb = 1; ntb <= kMaxNtb; ntb++) {
         if (!tile_fits(type, n_in, best.kg, ntb)) continue;
@@ -870,7 +873,7 @@ TileShape unsplit_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n
 // unsplit at 128). A requested count keeps two k groups, whose shares are the finer ones.
 TileShape linear_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_tok, uint32_t requested,
                        size_t workspace_bytes) {
-    const TileShape un = unsplit_shape(type, n_in, n_out, n_tok);
+    const TileShape un = unsplit_shape(type, n_in, n_out, n_tok, n_out <= kNarrowRows);
     if (requested == 1 || workspace_bytes <= kLinearCounterBytes) return un;
     const uint32_t cap = min(kMaxSplits, max(1u, n_in / 256));  // at least 256 elements a split
     TileShape best = un;
@@ -946,23 +949,28 @@ int launch_proj(uint32_t type, const void* const* W, const float* x, const float
         if (pro != kProNone || rope) return -2;
         if (epi != kEpiStore && epi != kEpiAccumulate && !pair) return -2;
         if (pair && (n_mats != 2 || n_out[0] != n_out[1])) return -1;
-        TileCall c{};
-        for (uint32_t m = 0; m < n_mats; m++) {
-            c.W[m] = static_cast<const uint8_t*>(W[m]);
-            c.out[m] = pair ? out[0] : out[m];
-            c.n_out[m] = n_out[m];
+        for (const bool narrow : {true, false}) {
+            TileCall c{};
+            uint32_t rows = 0;
+            for (uint32_t m = 0; m < n_mats; m++) {
+                if ((n_out[m] <= kNarrowRows) != narrow) continue;
+                c.W[c.n_mats] = static_cast<const uint8_t*>(W[m]);
+                c.out[c.n_mats] = pair ? out[0] : out[m];
+                c.n_out[c.n_mats++] = n_out[m];
+                rows += n_out[m];
+            }
+            if (rows == 0) continue;
+            c.x = x;
+            c.n_in = n_in;
+            c.n_tok = n_tok;
+            c.accumulate = epi == kEpiAccumulate;
+            c.pair = pair;
+            c.shape = unsplit_shape(type, n_in, rows, n_tok, narrow);
+            c.stream = stream;
+            const int rc = launch_tile_type(type, c);
+            if (rc != 0) return rc;
         }
-        c.n_mats = n_mats;
-        c.x = x;
-        c.n_in = n_in;
-        c.n_tok = n_tok;
-        c.accumulate = epi == kEpiAccumulate;
-        c.pair = pair;
-        uint32_t rows = 0;
-        for (uint32_t m = 0; m < n_mats; m++) rows += n_out[m];
-        c.shape = unsplit_shape(type, n_in, rows, n_tok);
-        c.stream = stream;
-        return launch_tile_type(type, c);
+        return 0;
     }
     MvArgs a{};
     if (epi == kEpiRopeKv) {

@@ -67,3 +67,26 @@ def test_ragged_end_reads_no_neighbour(dev, t):
     x = np.random.default_rng(4).standard_normal((n_tok, n_in)).astype(np.float32)
     got = _run(dev, t, raw, x, n_in, n_out, 0)
     assert np.all(np.isfinite(np.delete(got, 4, axis=1))) and not np.any(np.isfinite(got[:, 4]))
+
+
+@pytest.mark.parametrize("t", ["Q4_0", "F16"])
+@pytest.mark.parametrize("n_tok", [40, 130, 300])
+def test_chunk_of_narrow_and_wide_matrices(dev, t, n_tok):
+    """Matrices on both sides of the 4096 rows where the number of k groups changes, in one
+    ingot_proj call: each output equals ingot_linear (n_splits = 1) on its matrix bit for bit."""
+    import torch
+    import ingot_attn as ia
+
+    n_in, n_outs = 512, (4100, 96, 4096)
+    g = torch.Generator(device=dev)
+    g.manual_seed(n_tok)
+    x = torch.randn(n_tok, n_in, generator=g, device=dev)
+    ws = [torch.from_numpy(gb.random_weights(t, n, n_in, seed=n).reshape(-1)).to(dev) for n in n_outs]
+    outs = [torch.zeros(n_tok, n, device=dev) for n in n_outs]
+    refs = [torch.zeros(n_tok, n, device=dev) for n in n_outs]
+    ia.proj(ws, x, outs, ia.proj_desc(t, n_in, list(n_outs), n_tok=n_tok))
+    for w, r, n in zip(ws, refs, n_outs):
+        ia.linear(w, x, r, ia.linear_desc(t, n_in, n, n_tok, n_splits=1), use_workspace=False)
+    torch.cuda.synchronize()
+    for o, r in zip(outs, refs):
+        assert torch.equal(o, r) and bool(torch.isfinite(o).all())
