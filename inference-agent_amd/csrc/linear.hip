@@ -154,6 +154,7 @@ struct MvArgs {
     const float* x;
     const float* aux;  // rmsnorm weights [n_in]
     uint32_t n_in, row_bytes;
+    uint32_t blocks;  // linear_stream_kernel: row blocks of the call (the grid may be smaller)
     float eps;
     // kEpiRopeKv
     const float* inv_freq;
@@ -463,36 +464,44 @@ __device__ __forceinline__ uint32_t xslot(uint32_t i) {
     return (c << 3) | ((i & 7) ^ ((c >> 1) & 7));
 }
 
-template <int T, int RPH, int PRO, int EPI, int NT>
+template <int T, int RPH, int PRO, int EPI, int NT, bool LOOP>
 __global__ __launch_bounds__(NT) void linear_stream_kernel(const MvArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     constexpr int NDW = Col<T>::ndw;
     constexpr int RPM = EPI == kEpiSiluGate ? RPH / 2 : RPH;  // rows of each matrix per half-wave
     const uint32_t tid = threadIdx.x, lane = tid % 64, hw = tid / 32, l32 = tid % 32;
-    uint32_t m = 0, blk = blockIdx.x;
-    if constexpr (EPI != kEpiSiluGate) {
-        if (blk >= a.blk_end[0]) m = blk >= a.blk_end[1] ? 2 : 1;
-        if (m > 0) blk -= a.blk_end[m - 1];
-    }
-    const uint32_t n_in = a.n_in, row_bytes = a.row_bytes, n_out = a.n_out[m];
+    const uint32_t n_in = a.n_in, row_bytes = a.row_bytes;
     constexpr uint32_t NHW = NT / 32;  // half-waves
-    const uint32_t row0 = blk * NHW * RPM;  // the workgroup's first row of matrix m
 
-    // This half-wave's rows: RPM of matrix m (and the same RPM of matrix m + 1 for the gate/up
-    // pair); rows past n_out read the last row and are not written.
-    const uint64_t wbase = (uint64_t(row0) * row_bytes) & ~uint64_t(15);
+    // The rows of block blk of the call: this half-wave's RPM rows of matrix m from row0 on (and
+    // the same RPM of matrix m + 1 for the gate/up pair); rows past n_out read the last row and are
+    // not written. With LOOP (many more blocks than the chip holds workgroups) a workgroup takes
+    // blocks blockIdx.x, blockIdx.x + gridDim.x, ... and stages x once for all of them.
+    uint32_t blk = blockIdx.x, m, n_out, row0;
     uint32_t roff[RPH];
-#pragma unroll
-    for (int i = 0; i < RPH; i++) {
-        const uint32_t r = min(row0 + hw * RPM + uint32_t(i % RPM), n_out - 1);
-        roff[i] = uint32_t(uint64_t(r) * row_bytes - wbase);
-    }
-    const uint64_t left = (uint64_t(n_out) * row_bytes - wbase + 3) & ~uint64_t(3);
-    const int nrec = int(left < 0x7fffffffu ? left : 0x7fffffffu);
     __amdgpu_buffer_rsrc_t rs[EPI == kEpiSiluGate ? 2 : 1];
-    rs[0] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.W[m] + wbase), 0, nrec, kBufferFlags);
-    if constexpr (EPI == kEpiSiluGate)
-        rs[1] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.W[1] + wbase), 0, nrec, kBufferFlags);
+    auto take_block = [&]() {
+        uint32_t local = blk;
+        m = 0;
+        if constexpr (EPI != kEpiSiluGate) {
+            if (local >= a.blk_end[0]) m = local >= a.blk_end[1] ? 2 : 1;
+            if (m > 0) local -= a.blk_end[m - 1];
+        }
+        n_out = a.n_out[m];
+        row0 = local * NHW * RPM;
+        const uint64_t wbase = (uint64_t(row0) * row_bytes) & ~uint64_t(15);
+#pragma unroll
+        for (int i = 0; i < RPH; i++) {
+            const uint32_t r = min(row0 + hw * RPM + uint32_t(i % RPM), n_out - 1);
+            roff[i] = uint32_t(uint64_t(r) * row_bytes - wbase);
+        }
+        const uint64_t left = (uint64_t(n_out) * row_bytes - wbase + 3) & ~uint64_t(3);
+        const int nrec = int(left < 0x7fffffffu ? left : 0x7fffffffu);
+        rs[0] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.W[m] + wbase), 0, nrec, kBufferFlags);
+        if constexpr (EPI == kEpiSiluGate)
+            rs[1] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.W[1] + wbase), 0, nrec, kBufferFlags);
+    };
+    take_block();
 
     const uint32_t ncols = n_in / 32, last = ncols - 1;
     const uint32_t nsteps = (ncols + 31) / 32;
@@ -547,9 +556,11 @@ __global__ __launch_bounds__(NT) void linear_stream_kernel(const MvArgs a) {
     for (uint32_t base = NT * kMvChunks; base < nchunks; base += NT * kMvChunks) stage_round(base, false);
     float* part = reinterpret_cast<float*>(smem + 16 * nchunks);  // [4] wave partials
     __syncthreads();
-    load(0, b0);
-    load(1, b1);
-    load(2, b2);
+    if constexpr (!LOOP) {
+        load(0, b0);
+        load(1, b1);
+        load(2, b2);
+    }
     if constexpr (PRO == kProRmsNorm) {
         // rmsnorm_kernel's arithmetic and order: its 256 threads' float4 sums strided by 1024
         // elements (the first four waves here), row sums, the four wave partials in fixed
@@ -573,8 +584,6 @@ __global__ __launch_bounds__(NT) void linear_stream_kernel(const MvArgs a) {
     }
 
     float acc[RPH];
-#pragma unroll
-    for (int i = 0; i < RPH; i++) acc[i] = 0.f;
     auto compute = [&](uint32_t step, const uint32_t (&b)[RPH][NDW]) {
         const uint32_t c0 = step * 32 + l32;
         const uint32_t c = min(c0, last);
@@ -600,6 +609,14 @@ __global__ __launch_bounds__(NT) void linear_stream_kernel(const MvArgs a) {
             acc[i] = __fadd_rn(acc[i], valid ? v : 0.f);
         }
     };
+    for (;;) {
+    if constexpr (LOOP) {
+        load(0, b0);
+        load(1, b1);
+        load(2, b2);
+    }
+#pragma unroll
+    for (int i = 0; i < RPH; i++) acc[i] = 0.f;
     // three columns in flight (all of a 3072-long row), refilled as each is computed; the
     // last three buffered columns are computed without refills
     uint32_t st = 0;
@@ -663,22 +680,29 @@ __global__ __launch_bounds__(NT) void linear_stream_kernel(const MvArgs a) {
             }
         }
     }
+    blk += gridDim.x;
+    if (!LOOP || blk >= a.blocks) break;
+    take_block();
+    }
 }
 
-template <int T, int RPH, int PRO, int EPI, int NT>
+template <int T, int RPH, int PRO, int EPI, int NT, bool LOOP = false>
 int launch_st(const MvArgs& a, uint32_t blocks, size_t lds, hipStream_t stream) {
     static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&linear_stream_kernel<T, RPH, PRO, EPI, NT>),
+        reinterpret_cast<const void*>(&linear_stream_kernel<T, RPH, PRO, EPI, NT, LOOP>),
         hipFuncAttributeMaxDynamicSharedMemorySize, int(kMvLdsBytes));
     if (attr != hipSuccess) return -4;
-    hipLaunchKernelGGL((linear_stream_kernel<T, RPH, PRO, EPI, NT>), dim3(blocks), dim3(NT), lds, stream, a);
+    hipLaunchKernelGGL((linear_stream_kernel<T, RPH, PRO, EPI, NT, LOOP>), dim3(blocks), dim3(NT), lds, stream, a);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
 template <int T, int RPH, int PRO, int NT>
 int launch_st_epi(const MvArgs& a, int epi, uint32_t blocks, size_t lds, hipStream_t stream) {
     switch (epi) {
-        case kEpiStore: return launch_st<T, RPH, PRO, kEpiStore, NT>(a, blocks, lds, stream);
+        case kEpiStore:
+            if constexpr (NT == 256 && Fmt<T>::blk > 1)
+                if (blocks < a.blocks) return launch_st<T, RPH, PRO, kEpiStore, NT, true>(a, blocks, lds, stream);
+            return launch_st<T, RPH, PRO, kEpiStore, NT>(a, blocks, lds, stream);
         case kEpiAccumulate: return launch_st<T, RPH, PRO, kEpiAccumulate, NT>(a, blocks, lds, stream);
         case kEpiRopeKv:
             if constexpr (RPH >= 2) return launch_st<T, RPH, PRO, kEpiRopeKv, NT>(a, blocks, lds, stream);
@@ -720,7 +744,18 @@ int launch_stream_t(MvArgs a, uint32_t n_mats, int pro, int epi, hipStream_t str
     for (int r = kMaxRph; r >= min_rph && !nt; r /= 2)
         if (count(256, r, false) >= 256 || r == min_rph) { nt = 256; rph = r; }
     if (!nt) { nt = 256; rph = min_rph; }  // (Q6_K pairs: min_rph above kMaxRph)
-    const uint32_t blocks = count(nt, rph, true);
+    a.blocks = count(nt, rph, true);
+    // A block-quantized call of more row blocks than the chip holds workgroups (a vocabulary) loops
+    // over them: staging and normalizing x otherwise costs each workgroup as much as its rows.
+    // Logits of 128256 x 3072 (rmsnorm), 16032 / 4008 blocks on 2048 workgroups: Q6_K 101.0 -> 82.9
+    // us, Q4_0 56.0 -> 47.3, Q8_0 90.8 -> 80.1 (1024: 86.1, 48.3, 79.7; 512: 95.8, 49.1, 82.5); F16
+    // rows gain nothing (134.5, 136.0).
+    constexpr uint32_t kLoopGrid = 2048;
+    uint32_t blocks = a.blocks;
+    if (Fmt<T>::blk > 1 && nt == 256 && epi == kEpiStore && blocks > kLoopGrid) {
+        const uint32_t turns = (blocks + kLoopGrid - 1) / kLoopGrid;
+        blocks = (blocks + turns - 1) / turns;
+    }
     const size_t lds = size_t(a.n_in) * 4 * (pro == kProRmsNorm ? 2 : 1) + 16;
     if (lds > kMvLdsBytes) return -2;
     auto go = [&](auto pro_tag, auto nt_tag) -> int {

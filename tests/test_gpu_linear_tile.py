@@ -90,3 +90,30 @@ def test_chunk_of_narrow_and_wide_matrices(dev, t, n_tok):
     torch.cuda.synchronize()
     for o, r in zip(outs, refs):
         assert torch.equal(o, r) and bool(torch.isfinite(o).all())
+
+
+@pytest.mark.parametrize("t", ["Q4_0", "Q4_1", "Q8_0", "Q6_K"])
+@pytest.mark.parametrize("n_out", [16384, 66000])
+def test_one_token_many_rows(dev, oracle_mod, t, n_out):
+    """One token over more row blocks than the grid holds (each workgroup loops over several, the
+    last ones ragged), against the f32 oracle (bar of test_gpu_linear), plain and with the norm."""
+    import torch
+    import ingot_attn as ia
+
+    n_in = 256
+    n_out += 5
+    raw = gb.random_weights(t, n_out, n_in, seed=n_out)
+    rng = np.random.default_rng(7)
+    x, nw = rng.standard_normal((1, n_in)).astype(np.float32), np.ones(n_in, np.float32)
+    w, xd = torch.from_numpy(raw.reshape(-1)).to(dev), torch.from_numpy(x).to(dev)
+    for norm in (False, True):
+        out = torch.full((n_out + 16,), float("nan"), device=dev)
+        d = ia.proj_desc(t, n_in, [n_out], prologue=ia.PROJ_RMSNORM if norm else ia.PROJ_X, eps=1e-5)
+        ia.proj([w], xd, [out], d, norm_w=torch.from_numpy(nw).to(dev))
+        torch.cuda.synchronize()
+        xr = (x / np.sqrt((x.astype(np.float64) ** 2).mean() + 1e-5)).astype(np.float32) if norm else x
+        want = oracle_mod.linear(t, raw, xr, n_in, n_out)[0]
+        got = out.cpu().numpy()
+        dd = np.abs(got[:n_out] - want)
+        assert np.all(np.isnan(got[n_out:])) and np.all(np.isfinite(dd))
+        assert dd.max() <= 1e-5 * np.abs(want).max() + 1e-6 and np.linalg.norm(dd) <= 1e-5 * np.linalg.norm(want)
