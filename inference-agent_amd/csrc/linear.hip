@@ -853,25 +853,29 @@ int launch_tile_type(uint32_t type, const TileCall& c) {
     }
 }
 
-// Measured time of one workgroup over 3072 elements of n_in beside its fixed part of ~4 us
-// (Q4_0, us): [k groups 4, 2, 1][token blocks of 32].
+// Measured time of one workgroup over 3072 elements of n_in beside its fixed part of ~4 us (us):
+// [k groups 4, 2, 1][token blocks of 32], of Q4_0 (the other types are near it in proportion) and of
+// Q6_K, whose dequantization weighs more against the token blocks. 0: no such kernel.
 constexpr uint32_t kMaxSplits = 8, kMaxNtb = 4;
-float tile_walk_us(uint32_t kg, uint32_t ntb) {
-    constexpr float t[3][kMaxNtb + 1] = {{0, 9, 13, 19, 0}, {0, 0, 20, 25, 31}, {0, 0, 30, 40, 50}};
-    return t[kg == 4 ? 0 : kg == 2 ? 1 : 2][ntb];
+float tile_walk_us(uint32_t type, uint32_t kg, uint32_t ntb) {
+    constexpr float t[2][3][kMaxNtb + 1] = {{{0, 9, 13, 19, 0}, {0, 0, 20, 25, 31}, {0, 0, 30, 40, 50}},
+                                            {{0, 18, 24, 30, 0}, {0, 0, 40, 45, 48}, {0, 0, 60, 68, 77}}};
+    return t[type == kQ6_K][kg == 4 ? 0 : kg == 2 ? 1 : 2][ntb];
 }
 
 bool tile_fits(uint32_t type, uint32_t n_in, uint32_t kg, uint32_t ntb) {
-    if (tile_walk_us(kg, ntb) == 0) return false;
-    if (type == kF32 && kg == 4 && ntb == 3) return false;           // (its weights' LDS leaves no room)
+    if (tile_walk_us(type, kg, ntb) == 0) return false;
+    // F32: the weights' LDS leaves no room for 3 blocks on four k groups, their registers none for 4
+    // (they spill: gate/up at 512 tokens 180.7 us).
+    if (type == kF32 && (ntb == 4 || (kg == 4 && ntb == 3))) return false;
     return ntb <= 2 || uint64_t(128) * ntb * n_in < 0x80000000ull;  // 32-bit offsets into a tile's x
 }
 
 // Estimated time (us) of a shape: rounds of 256 workgroups, each its share of n_in, then the tail
 // of a split: the last workgroup of a tile reads every split's partial tile (~32 KB a us).
-float tile_us(uint32_t n_in, uint64_t tiles, const TileShape& s) {
+float tile_us(uint32_t type, uint32_t n_in, uint64_t tiles, const TileShape& s) {
     const float rounds = float((tiles * s.splits + 255) / 256);
-    const float t = rounds * (4.f + tile_walk_us(s.kg, s.ntb) * float(n_in) / float(3072 * s.splits));
+    const float t = rounds * (4.f + tile_walk_us(type, s.kg, s.ntb) * float(n_in) / float(3072 * s.splits));
     return s.splits == 1 ? t : t + 3.f + float(s.splits * tile_bytes(s)) / 32768.f;
 }
 
@@ -896,7 +900,7 @@ TileShape unsplit_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n
     for (uint32_t ntb = 1; ntb <= kMaxNtb; ntb++) {
         if (!tile_fits(type, n_in, best.kg, ntb)) continue;
         const TileShape s{ntb, best.kg, 1};
-        const float u = tile_us(n_in, tile_count(n_out, n_tok, s), s);
+        const float u = tile_us(type, n_in, tile_count(n_out, n_tok, s), s);
         if (best.ntb == 0 || u < t) { best.ntb = ntb; t = u; }
     }
     return best;
@@ -912,7 +916,7 @@ TileShape linear_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_
     if (requested == 1 || workspace_bytes <= kLinearCounterBytes) return un;
     const uint32_t cap = min(kMaxSplits, max(1u, n_in / 256));  // at least 256 elements a split
     TileShape best = un;
-    float t = tile_us(n_in, tile_count(n_out, n_tok, un), un);
+    float t = tile_us(type, n_in, tile_count(n_out, n_tok, un), un);
     bool split = false;
     for (uint32_t kg = 4; kg >= 1; kg /= 2) {
         if (requested > 1 && kg != 2) continue;
@@ -925,7 +929,7 @@ TileShape linear_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_
                 const uint64_t tiles = tile_count(n_out, n_tok, s);
                 const bool fits = s.splits == 1 ||
                     (tiles <= kLinearMaxTiles && kLinearCounterBytes + tiles * s.splits * tile_bytes(s) <= workspace_bytes);
-                const float u = tile_us(n_in, tiles, s);
+                const float u = tile_us(type, n_in, tiles, s);
                 const bool must = (requested > 1 || n_tok <= 128) && s.splits > 1;  // a split is wanted
                 if (fits && ((must && !split) || (must == split && u < t))) {
                     best = s;
