@@ -290,7 +290,7 @@ ENVELOPE_DECODE = (("decode-64/8-hd128-4096", 64, 8, 128, 4096),
 ENVELOPE_PREFILL = (("prefill-32/8-hd128-512@3584", 32, 8, 128, 3584, 512),
                     ("prefill-32/8-hd64-512@3584", 32, 8, 64, 3584, 512),
                     ("prefill-16/8-hd256-512@3584", 16, 8, 256, 3584, 512),
-                    ("prefill-24/8-hd96-128@0", 24, 8, 96, 0, 128))  # the fallback kernel
+                    ("prefill-24/8-hd96-128@0", 24, 8, 96, 0, 128))  # the MFMA kernel, f32 accuracy
 
 
 def envelope(torch, ia, steps, warmup, use_graph):
