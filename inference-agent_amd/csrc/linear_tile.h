@@ -45,6 +45,14 @@ constexpr size_t tile_lds(uint32_t ntb, uint32_t kg, size_t w) {
 }
 constexpr size_t tile_bytes(const TileShape& s) { return size_t(tile_rows(s.kg)) * s.ntb * 32 * 4; }
 
+// First token block (32 tokens) of token tile tt: the nb blocks spread evenly over tiles_m tiles, the
+// first nb % tiles_m of them one block longer. (tt * nb / tiles_m would pass 32 bits from 2.1 million
+// tokens of one-block tiles, 4.2 million of four-block tiles on.)
+constexpr uint32_t tile_block0(uint32_t tt, uint32_t nb, uint32_t tiles_m) {
+    const uint32_t longer = nb % tiles_m;
+    return tt * (nb / tiles_m) + (tt < longer ? tt : longer);
+}
+
 // 0, -1 (grid too large or a bad shape) or -4 (launch failed). T: the GGUF type id.
 template <int T> int launch_tile(const TileCall& c);
 

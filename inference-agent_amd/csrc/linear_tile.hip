@@ -181,7 +181,7 @@ void linear_tile_kernel(const TileArgs a) {
     const uint32_t rowbase = rtl * RT + (PAIR ? rg % (RG / 2) : rg) * 32;  // the wave's rows
     // The token blocks are spread evenly over the token tiles.
     const uint32_t nb = (a.n_tok + 31) / 32;
-    const uint32_t tb0 = tt * nb / a.tiles_m, tb1 = (tt + 1) * nb / a.tiles_m;
+    const uint32_t tb0 = tile_block0(tt, nb, a.tiles_m), tb1 = tile_block0(tt + 1, nb, a.tiles_m);
     const uint32_t tok0 = 32 * tb0, toks = min(a.n_tok - tok0, 32 * (tb1 - tb0));
 
     // This split's elements, in units of KG * unit; each k group takes a contiguous share, U steps

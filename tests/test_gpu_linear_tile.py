@@ -117,3 +117,23 @@ def test_one_token_many_rows(dev, oracle_mod, t, n_out):
         dd = np.abs(got[:n_out] - want)
         assert np.all(np.isnan(got[n_out:])) and np.all(np.isfinite(dd))
         assert dd.max() <= 1e-5 * np.abs(want).max() + 1e-6 and np.linalg.norm(dd) <= 1e-5 * np.linalg.norm(want)
+
+
+def test_millions_of_tokens(dev):
+    """Above 4.2 million tokens a product of token tile and token block count passes 32 bits: every
+    row of out is written, and accumulated into, once (checked against torch in f32, both operands
+    rounded to f16: only the order of 32 f32 products differs)."""
+    import torch
+    import ingot_attn as ia
+
+    n_tok, n_in, n_out = 4_194_304 + 33, 32, 32
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    x = torch.randn(n_tok, n_in, generator=g, device=dev)
+    w = (torch.randn(n_out, n_in, generator=g, device=dev) / n_in ** 0.5).half()
+    want = x.half().float() @ w.float().t()
+    out = torch.full((n_tok, n_out), float("nan"), device=dev)
+    for acc in (False, True):
+        ia.linear(w.view(torch.uint8).reshape(-1), x, out, ia.linear_desc("F16", n_in, n_out, n_tok, accumulate=acc))
+        d = (out - want * (2 if acc else 1)).abs().max()
+        assert bool(torch.isfinite(out).all()) and float(d) <= 1e-5 * float(want.abs().max()) * 2
