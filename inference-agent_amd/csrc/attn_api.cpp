@@ -236,9 +236,11 @@ size_t ingot_attn_decode_workspace_size(const IngotAttnDecodeDesc* d) {
 
 // Whether a head size without a kernel of its own prefills on the MFMA kernel with f32 accuracy
 // (24 Q / 8 KV heads of 96, 301 tokens at 211: 82 us a call on the fallback kernel, 13 on the MFMA
-// one, whose 16-byte chunks of a cache row need a multiple of 8).
+// one, whose 16-byte chunks of a cache row need a multiple of 8, and whose 64 q and out rows of a
+// block lie within the 2 GiB of a descriptor's 32-bit offsets: rows further apart stay on the
+// fallback kernel's 64-bit addresses, as 64-bit ones in the MFMA kernel cost every call 2-7%).
 bool exact_prefill(const IngotAttnPrefillDesc* d) {
-    return d->head_dim % 8 == 0 && d->head_dim < 256;
+    return d->head_dim % 8 == 0 && d->head_dim < 256 && d->q_stride <= 0x7fffffffu / (64 * sizeof(float));
 }
 
 size_t ingot_attn_prefill_workspace_size(const IngotAttnPrefillDesc* d) {

@@ -56,3 +56,26 @@ def test_zero_filled_dims(dev, hd, nh, nkv, pos, n, pad, gain, bar):
         want = p / p.sum(1, keepdims=True) @ v[L:, c].astype(np.float64)
         d = got[:, h * hd:(h + 1) * hd] - want
         assert np.all(np.isfinite(d)) and np.linalg.norm(d) <= bar * np.linalg.norm(want), f"head {h}"
+
+
+def test_rows_beyond_2gib(dev):
+    """Rows of q and out so far apart that a block of 64 tokens spans more than 2 (and 4) GiB: the
+    same values as from dense rows, up to f32 rounding (such calls run the fallback kernel)."""
+    import torch
+    import ingot_attn as ia
+
+    hd, nh, nkv, pos, n = 96, 3, 1, 40, 64
+    g = torch.Generator(device=dev)
+    g.manual_seed(1)
+    q = torch.randn(n, nh * hd, generator=g, device=dev)
+    k = torch.randn(pos + n, nkv * hd, generator=g, device=dev).half()
+    v = torch.randn(pos + n, nkv * hd, generator=g, device=dev).half()
+    want = torch.empty_like(q)
+    ia.attn_prefill(q, k, v, want, ia.prefill_desc(nh, nkv, hd, pos, n))
+    for stride in (8_388_607, 8_388_608, 9_000_003, 18_000_000):
+        far, out = (torch.zeros(n, stride, device=dev) for _ in range(2))
+        far[:, : nh * hd] = q
+        ia.attn_prefill(far, k, v, out, ia.prefill_desc(nh, nkv, hd, pos, n, q_stride=stride))
+        assert float((out[:, : nh * hd] - want).norm() / want.norm()) <= 2e-6, stride
+        assert not bool(out[:, nh * hd:].any()), "wrote past the heads"
+        del far, out
