@@ -53,6 +53,7 @@ typedef __attribute__((address_space(3))) half8 lds_half8;
 
 // Keys per tile: 64, or 32 for head_dim 256 (four 64 KB stages would not fit the LDS).
 template <int HD> constexpr int kBN = HD == 256 ? 32 : 64;
+constexpr float kLazyExact = 5.f, kExactHi = 1024.f, kExactLo = 4096.f;  // EXACT: its headroom, scales of P's parts
 constexpr float kLazy = 8.f;                   // base-2 headroom before the reference max moves
 constexpr int kBufferFlags = 0x00020000;       // buffer descriptor word 3 (raw, 32-bit format)
 constexpr int kScDevice = 16;                  // buffer cache-policy bits: sc1 = device scope
@@ -89,13 +90,22 @@ template <int HD> __device__ __forceinline__ int swz_v(int row) {
 
 // EXACT: head sizes without a kernel of their own (hd < HD, a multiple of 8), one head per unit,
 // never split: the dims past hd are zero in LDS and not stored, and q and the probabilities enter
-// the MFMAs as two f16 parts each (hi + lo, together ~22 bits; K and V are f16 as stored), so that
-// the scores and the sums keep the f32 accuracy of the fallback kernel at twice the matrix work.
+// the MFMAs as two f16 parts each (together ~22 bits; K and V are f16 as stored), so that the scores
+// and the sums keep the f32 accuracy of the fallback kernel at twice the matrix work. f16 has no
+// exponents for small probabilities, so P's parts are scaled apart: p <= 2^5 of the reference
+// maximum, hi = f16(2^10 p), lo = f16(2^12 (2^10 p - hi)): a relative 2^-22 from p = 2^-24 on, an
+// absolute 2^-47 below. Measured against 64 bits with all the weight on a key whose V row is zero,
+// the others g nats below it (head size 96, 2048 keys; fallback kernel / here): g = 8 4.3e-7 /
+// 3.0e-7, 16 6.9e-7 / 6.3e-7, 20 9.0e-7 / 9.0e-7, 24 1.1e-6 / 2.8e-5 (unscaled: 1.3e-5, 4e-2 and all
+// wrong from there). lo's sums stand apart in their own accumulators, or, where registers do not
+// hold both (head sizes above 128 would spill: 64 tokens at 4000, 111 -> 200 us), in O, which is
+// then held times 2^12 and takes hi by an fma.
 // A query row is first scaled by a power of two that puts its largest element at 2^8..2^9 (any
 // finite q then fits the f16 parts, and a small one keeps its low bits); the scores are scaled
 // back in f32. Bound by the LDS reads and the chain of the longest key walk, like a short chunk of
 // a 128-wide head: 24 / 8 heads of 96, 301 tokens at 211, 82 -> 13 us (154 TFLOP/s of useful
-// products), error against 64 bits 3.6e-7 -> 2.4e-7.
+// products), error against 64 bits 3.4e-7 -> 2.3e-7 (head size 192, 500 tokens at 4000: 6.1e-7 ->
+// 4.3e-7).
 template <int HD, int G, int QW, int KG, bool EXACT = false>
 __global__ __launch_bounds__(64 * QW * KG) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict__ K,
@@ -105,6 +115,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
     static_assert(!EXACT || G == 1, "one head per unit");
     const uint32_t hd = EXACT ? hd_ : HD;
     constexpr int GQ = EXACT ? 2 : G;  // f16 rows of q per query: the unit's heads, or hi and lo
+    constexpr float kHead = EXACT ? kLazyExact : kLazy;
     constexpr int BN = kBN<HD>, RB = kRowBytes<HD>, CPR = kChunks<HD>, TB = kTileBytes<HD>, SB = kStageBytes<HD>;
     constexpr int HALVES = BN / 32;  // 32-key halves per tile
     constexpr int PB = HD * 2 + 16;  // bytes per split record: o[HD] / l as f16, then {m, l, 0, 0}
@@ -282,6 +293,9 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
     // keys), so P = 2^S' <= 2^kLazy and the O rescale is rare. O/l does not depend on the
     // reference, so this is exact.
     float4v O[G][ND];
+    // EXACT: the sums of P's lo parts, times kExactLo (in O itself without LO).
+    constexpr bool LO = EXACT && HD <= 128;
+    float4v Olo[LO ? ND : 1];
     float m[G], l[G];
     float4v negm[G];  // {-m, -m, -m, -m}: the C operand of the first score MFMA of each tile
     bool started[G];
@@ -293,7 +307,10 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
         negm[h] = float4v{0.f, 0.f, 0.f, 0.f};
         started[h] = false;
 #pragma unroll
-        for (int d = 0; d < ND; d++) O[h][d] = float4v{0.f, 0.f, 0.f, 0.f};
+        for (int d = 0; d < ND; d++) {
+            O[h][d] = float4v{0.f, 0.f, 0.f, 0.f};
+            if constexpr (LO) Olo[d] = float4v{0.f, 0.f, 0.f, 0.f};
+        }
     }
 
     // `dma(k)` issues copy instruction k of the next tile (k < kInstPerWave).
@@ -358,7 +375,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
 #pragma unroll
                     for (int T = 0; T < 2; T++)
                         x = fmaxf(x, fmaxf(fmaxf(S[T][h][0], S[T][h][1]), fmaxf(S[T][h][2], S[T][h][3])));
-                need = __builtin_amdgcn_ballot_w64(x > kLazy) != 0;
+                need = __builtin_amdgcn_ballot_w64(x > kHead) != 0;
             }
             if (need) {  // wave-uniform, rare after warm-up
                 bool pending = false;
@@ -367,7 +384,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
                     float x = fmaxf(fmaxf(fmaxf(S[0][h][0], S[0][h][1]), fmaxf(S[0][h][2], S[0][h][3])),
                                     fmaxf(fmaxf(S[1][h][0], S[1][h][1]), fmaxf(S[1][h][2], S[1][h][3])));
                     x = max_lanes4(x);  // max over the 4 lanes of a query
-                    const bool grow = started[h] ? (x > kLazy) : (x > -__builtin_inff());
+                    const bool grow = started[h] ? (x > kHead) : (x > -__builtin_inff());
                     const float delta = grow ? x : 0.f;
                     // (a first maximum may be far below 0: nothing is accumulated yet to rescale)
                     const float alpha = started[h] ? fast_exp2(-delta) : 0.f;
@@ -379,7 +396,10 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
 #pragma unroll
                     for (int T = 0; T < 2; T++) S[T][h] -= delta;
 #pragma unroll
-                    for (int d = 0; d < ND; d++) O[h][d] *= alpha;
+                    for (int d = 0; d < ND; d++) {
+                        O[h][d] *= alpha;
+                        if constexpr (LO) Olo[d] *= alpha;
+                    }
                 }
                 all_started = __builtin_amdgcn_ballot_w64(pending) == 0;
             }
@@ -392,13 +412,22 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         const float p = fast_exp2(S[T][h][j]);
-                        P[h][4 * T + j] = _Float16(p);
-                        if constexpr (EXACT) {
-                            P[1][4 * T + j] = _Float16(p - float(P[0][4 * T + j]));
-                            S[T][0][j] = p;
-                        }
+                        if constexpr (EXACT) S[T][0][j] = p;
+                        else P[h][4 * T + j] = _Float16(p);
                     }
-                if constexpr (EXACT) {  // (the eight summed first: a shorter chain of roundings)
+                if constexpr (EXACT) {
+                    // (v_fma_mixlo / mixhi: a product with one rounding to f16 each)
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const float p0 = S[e / 4][0][e % 4], p1 = S[e / 4][0][e % 4 + 1];
+                        half2v hi = {_Float16(fmaf(p0, kExactHi, 0.f)), _Float16(fmaf(p1, kExactHi, 0.f))};
+                        asm("" : "+v"(hi));  // (else every product is formed a second time for the part below)
+                        P[0][e] = hi[0];
+                        P[0][e + 1] = hi[1];
+                        P[1][e] = _Float16(fmaf(fmaf(p0, kExactHi, -float(hi[0])), kExactLo, 0.f));
+                        P[1][e + 1] = _Float16(fmaf(fmaf(p1, kExactHi, -float(hi[1])), kExactLo, 0.f));
+                    }
+                    // (the eight summed first: a shorter chain of roundings)
                     l[0] += ((S[0][0][0] + S[0][0][1]) + (S[0][0][2] + S[0][0][3])) +
                             ((S[1][0][0] + S[1][0][1]) + (S[1][0][2] + S[1][0][3]));
                     break;
@@ -428,8 +457,16 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
                 }
                 const half8 a = __builtin_shufflevector(part_[0], part_[1], 0, 1, 2, 3, 4, 5, 6, 7);
                 if constexpr (EXACT) {  // (32 keys summed on their own, then one rounding into O)
-                    float4v t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, Pp[1], float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    O[0][d] += __builtin_amdgcn_mfma_f32_16x16x32_f16(a, Pp[0], t, 0, 0, 0);
+                    const float4v zero = {0.f, 0.f, 0.f, 0.f};
+                    const float4v hi = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, Pp[0], zero, 0, 0, 0);
+                    if constexpr (LO) {
+                        Olo[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, Pp[1], Olo[d], 0, 0, 0);
+                        O[0][d] += hi;
+                    } else {  // (O is held times kExactLo)
+                        O[0][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, Pp[1], O[0][d], 0, 0, 0);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) O[0][d][e] = fmaf(hi[e], kExactLo, O[0][d][e]);
+                    }
                     continue;
                 }
 #pragma unroll
@@ -519,6 +556,10 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
         }
     }
 
+    if constexpr (LO)
+#pragma unroll
+        for (int d = 0; d < ND; d++) O[0][d] += Olo[d] * (1.f / kExactLo);
+
     if (KG == 2) {
         // Merge the two key groups through LDS (the tiles are no longer read): group 1 stores
         // its (O, m, l, started) per lane for every head, one barrier, group 0 folds them in
@@ -583,7 +624,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
 #pragma unroll
         for (int h = 0; h < G; h++) {
             const uint32_t head = kvh * G + h;
-            const float inv = l[h] > 0.f ? 1.f / l[h] : 0.f;
+            const float inv = (l[h] > 0.f ? 1.f / l[h] : 0.f) * (EXACT ? 1.f / (LO ? kExactHi : kExactHi * kExactLo) : 1.f);
             const int off = int(4 * ((row - qblk0) * q_stride + head * hd + 4 * g));
 #pragma unroll
             for (int d = 0; d < ND; d++)

@@ -1,6 +1,6 @@
 """Prefill at head sizes that share the MFMA kernel with zero-filled dims (multiples of 8 below 256
 other than 64 and 128): against a float64 reference on the CPU. q and the probabilities enter as
-two f16 parts (a relative 2^-22 each), sums are f32: with scores of magnitude s the result is off by
+two f16 parts (a relative 2^-22 each, the probabilities down to 2^-24), sums are f32: with scores of magnitude s the result is off by
 about (s + 4) * 2^-22, so rel-L2 <= 2e-6 at s ~ 4 and <= 2e-5 at s ~ 100 (the first maximum of a
 key group may then lie far below zero)."""
 from __future__ import annotations
@@ -79,3 +79,41 @@ def test_rows_beyond_2gib(dev):
         assert float((out[:, : nh * hd] - want).norm() / want.norm()) <= 2e-6, stride
         assert not bool(out[:, nh * hd:].any()), "wrote past the heads"
         del far, out
+
+
+@pytest.mark.parametrize("hd", [40, 96, 136])
+@pytest.mark.parametrize("where", ["first", "last"])
+@pytest.mark.parametrize("gap,bar", [(8.0, 2e-6), (12.0, 2e-6), (16.0, 2e-6), (20.0, 4e-6), (24.0, 2e-4)])
+def test_small_probabilities(dev, hd, where, gap, bar):
+    """An attention sink: one key `gap` nats above the others' mean score, with a zero V row, so that
+    the output is made of probabilities around e^-gap alone. They are held to a relative 2^-22 down to
+    2^-24 and the scores (up to 1.44 gap in the exponent of 2) rounded to f32, about 1.44 * 24 *
+    2^-25 * ln 2 = 7e-7: rel-L2 <= 2e-6, the bar of ordinary scores. Below 2^-24 (gap 16.6) the
+    probabilities keep an absolute 2^-47 of the largest: at e^-20 2^-18 (4e-6), at e^-24 2^-12 (2e-4)."""
+    import torch
+    import ingot_attn as ia
+
+    nh, nkv, pos, n = 2, 1, 2000, 48
+    L, kvd = pos + n, nkv * hd
+    rng = np.random.default_rng(int(gap) + hd)
+    at = 0 if where == "first" else pos  # (visible to every query)
+    q = rng.standard_normal((n, nh * hd)).astype(np.float32)
+    k = rng.standard_normal((L, kvd)).astype(np.float16)
+    v = rng.standard_normal((L, kvd)).astype(np.float16)
+    # dimension 0 carries the sink's score: q = 8 there, the sink's k such that 8 k / sqrt(hd) = gap
+    q[:, ::hd] = 8.0
+    k[:, 0], k[at] = 0, 0
+    k[at, 0] = gap * np.sqrt(hd) / 8.0
+    v[at] = 0
+    t = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+    out = torch.empty(n, nh * hd, device=dev)
+    ia.attn_prefill(t(q), t(k), t(v), out, ia.prefill_desc(nh, nkv, hd, pos, n))
+    got = out.cpu().numpy()
+    for h in range(nh):
+        c = slice(h * hd, (h + 1) * hd)
+        s = q[:, c].astype(np.float64) @ k.astype(np.float64).T * np.float64(np.float32(1.0 / np.sqrt(hd)))
+        s[np.arange(L)[None, :] > pos + np.arange(n)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        want = p / p.sum(1, keepdims=True) @ v.astype(np.float64)
+        rel = np.linalg.norm(got[:, c] - want) / np.linalg.norm(want)
+        assert rel <= bar
