@@ -101,8 +101,8 @@ template <int HD> __device__ __forceinline__ int swz_v(int row) {
 // hold both (head sizes above 128 would spill: 64 tokens at 4000, 111 -> 200 us), in O, which is
 // then held times 2^12 and takes hi by an fma.
 // A query row is first scaled by a power of two that puts its largest element at 2^8..2^9 (any
-// finite q then fits the f16 parts, and a small one keeps its low bits); the scores are scaled
-// back in f32. Bound by the LDS reads and the chain of the longest key walk, like a short chunk of
+// finite q then fits the f16 parts, and one down to 2^-100 keeps its low bits); the scores are scaled
+// back, and by scale * log2(e), in f32. Bound by the LDS reads and the chain of the longest key walk, like a short chunk of
 // a 128-wide head: 24 / 8 heads of 96, 301 tokens at 211, 82 -> 13 us (154 TFLOP/s of useful
 // products), error against 64 bits 3.4e-7 -> 2.3e-7 (head size 192, 500 tokens at 4000: 6.1e-7 ->
 // 4.3e-7).
@@ -223,7 +223,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
     constexpr int NT = 64 * QW * KG;
     constexpr int kQIt = (kF4 + NT - 1) / NT;
     float4v qx[kQIt];
-    __shared__ float qback[EXACT ? QW * 16 : 1];  // per query: the power of two that scales its scores back
+    __shared__ float qback[EXACT ? QW * 16 : 1];  // per query: what its scores are multiplied by
     {
         const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<float*>(q + size_t(qblk0) * q_stride + size_t(kvh) * G * hd), 0,
@@ -255,10 +255,9 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
             float x = fmaxf(fmaxf(fabsf(qx[it][0]), fabsf(qx[it][1])), fmaxf(fabsf(qx[it][2]), fabsf(qx[it][3])));
 #pragma unroll
             for (int o = 1; o < QF4; o <<= 1) x = fmaxf(x, __shfl_xor(x, o));
-            const int e = 8 - min(max(int(__float_as_uint(x * qscale) >> 23) - 127, -100), 100);
-            unit = 1.f;
-            qx[it] = qx[it] * qscale * ldexpf(1.f, e);
-            if (c4 == 0) qback[ql] = ldexpf(1.f, -e);
+            const int e = 8 + 127 - max(int(__float_as_uint(x) >> 23), 127 - 100);
+            unit = __uint_as_float(uint32_t(127 + e) << 23);  // 2^e, e = -120 .. 108
+            if (c4 == 0) qback[ql] = __uint_as_float(uint32_t(127 - e) << 23) * qscale;
         }
 #pragma unroll
         for (int e = 0; e < 4; e++) {

@@ -117,3 +117,27 @@ def test_small_probabilities(dev, hd, where, gap, bar):
         want = p / p.sum(1, keepdims=True) @ v.astype(np.float64)
         rel = np.linalg.norm(got[:, c] - want) / np.linalg.norm(want)
         assert rel <= bar
+
+
+@pytest.mark.parametrize("hd", [8, 96, 200])
+@pytest.mark.parametrize("size", [1e-38, 1e-30, 1e30, 3e32, 1e35])
+def test_any_finite_query(dev, hd, size):
+    """Queries of any finite size: the softmax of the tiny ones is uniform, of the huge ones all on
+    one key (test and reference agree on which: the best score leads by far more than f32 rounding)."""
+    import torch
+    import ingot_attn as ia
+
+    n = 40
+    rng = np.random.default_rng(hd)
+    k = rng.standard_normal((n, hd)).astype(np.float16)
+    v = rng.standard_normal((n, hd)).astype(np.float16)
+    q = (rng.standard_normal((n, hd)) * size).astype(np.float32)
+    t = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+    out = torch.empty(n, hd, device=dev)
+    ia.attn_prefill(t(q), t(k), t(v), out, ia.prefill_desc(1, 1, hd, 0, n))
+    s = q.astype(np.float64) @ k.astype(np.float64).T / np.sqrt(hd)
+    s[np.arange(n)[None, :] > np.arange(n)[:, None]] = -np.inf
+    p = np.exp(s - s.max(1, keepdims=True))
+    want = p / p.sum(1, keepdims=True) @ v.astype(np.float64)
+    got = out.cpu().numpy()
+    assert np.all(np.isfinite(got)) and np.linalg.norm(got - want) <= 2e-6 * np.linalg.norm(want)
