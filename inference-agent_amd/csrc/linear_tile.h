@@ -25,6 +25,7 @@ struct TileCall {
     TileShape shape;
     void* workspace;  // counters, then partial tiles (shape.splits > 1)
     hipStream_t stream;
+    uint32_t row0 = 0, rows = ~0u;  // the rows of each matrix to compute (out keeps its n_out columns)
 };
 
 // Rows per tile, k elements per stage and bytes of one partial tile of a shape.

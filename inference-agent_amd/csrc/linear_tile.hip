@@ -22,6 +22,8 @@
 // through LDS); a branch around the dequantization of a ragged end kept the compiler from
 // interleaving MFMAs with it (67 M wave-cycles, 52 M without); starting the token tiles at
 // different stages, as the L2 channels would like it, changed nothing.
+#include <algorithm>
+
 #include "linear_formats.h"
 #include "linear_tile.h"
 
@@ -145,7 +147,8 @@ __device__ __forceinline__ void col_read(const uint8_t* row, uint32_t off, uint3
 struct TileArgs {
     const uint8_t* W[3];
     float* out[3];
-    uint32_t n_out[3];
+    uint32_t n_out[3];     // rows [row0, n_out[m]) of matrix m, whose out has ld[m] columns
+    uint32_t ld[3], row0;
     uint32_t tile_end[2];  // row tiles of matrix m: [tile_end[m-1], tile_end[m])
     const float* x;
     uint32_t n_in, n_tok, row_bytes, accumulate;
@@ -177,8 +180,9 @@ void linear_tile_kernel(const TileArgs a) {
     const uint8_t* const W = mat == 0 ? a.W[0] : mat == 1 ? a.W[1] : a.W[2];
     float* const out = PAIR || mat == 0 ? a.out[0] : mat == 1 ? a.out[1] : a.out[2];
     const uint32_t n_out = PAIR || mat == 0 ? a.n_out[0] : mat == 1 ? a.n_out[1] : a.n_out[2];
+    const uint32_t ld = PAIR || mat == 0 ? a.ld[0] : mat == 1 ? a.ld[1] : a.ld[2];
     const uint32_t rtl = PAIR ? rt : rt - (mat == 0 ? 0u : mat == 1 ? a.tile_end[0] : a.tile_end[1]);
-    const uint32_t rowbase = rtl * RT + (PAIR ? rg % (RG / 2) : rg) * 32;  // the wave's rows
+    const uint32_t rowbase = a.row0 + rtl * RT + (PAIR ? rg % (RG / 2) : rg) * 32;  // the wave's rows
     // The token blocks are spread evenly over the token tiles.
     const uint32_t nb = (a.n_tok + 31) / 32;
     const uint32_t tb0 = tile_block0(tt, nb, a.tiles_m), tb1 = tile_block0(tt + 1, nb, a.tiles_m);
@@ -470,7 +474,7 @@ void linear_tile_kernel(const TileArgs a) {
     for (int b = 0; b < NTB; b++) {
         const uint32_t t = 32 * b + n;
         if (kg != uint32_t(b % KG) || t >= toks) continue;
-        float* o = out + size_t(tok0 + t) * n_out + rowbase + 4 * h;
+        float* o = out + size_t(tok0 + t) * ld + rowbase + 4 * h;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             const uint32_t r = rowbase + 8 * q + 4 * h;
@@ -504,13 +508,45 @@ int launch(const TileArgs& a, dim3 grid, hipStream_t stream) {
 template <int T>
 int launch_tile(const TileCall& c) {
     const uint32_t kg = c.shape.kg, ntb = c.shape.ntb;
+    // The kernel's offsets are 32 bits, below kOob: where a tile's tokens or a wave's 32 rows pass
+    // that (rows of 67 MB on), a call runs in pieces of fewer of them. The sums keep their order.
+    constexpr uint64_t kReach = 0x7ffffff0;
+    const uint64_t row_bytes = uint64_t(c.n_in) / Fmt<T>::blk * Fmt<T>::bytes, x_bytes = 4 * uint64_t(c.n_in);
+    const uint32_t longest = std::max(c.n_out[0], std::max(c.n_mats > 1 ? c.n_out[1] : 0, c.n_mats > 2 ? c.n_out[2] : 0));
+    if (x_bytes > kReach || row_bytes > kReach) return -1;
+    if (std::min(c.n_tok, 32 * ntb) * x_bytes > kReach) {
+        const uint32_t step = uint32_t(kReach / x_bytes);
+        for (uint32_t t = 0; t < c.n_tok; t += step) {
+            TileCall p = c;
+            p.x += size_t(t) * c.n_in;
+            p.n_tok = std::min(step, c.n_tok - t);
+            for (uint32_t m = 0; m < c.n_mats; m++) p.out[m] += size_t(t) * c.n_out[m];
+            const int rc = launch_tile<T>(p);
+            if (rc != 0) return rc;
+        }
+        return 0;
+    }
+    if (std::min(std::min(longest, c.rows), 32u) * row_bytes > kReach) {
+        const uint32_t step = uint32_t(kReach / row_bytes);
+        for (uint32_t r = 0; r < longest; r += step) {
+            TileCall p = c;
+            p.row0 = r;
+            p.rows = step;
+            const int rc = launch_tile<T>(p);
+            if (rc != 0) return rc;
+        }
+        return 0;
+    }
     TileArgs a{};
     const uint32_t rows = tile_rows(kg) / (c.pair ? 2 : 1);
+    a.row0 = c.row0;
     for (uint32_t m = 0; m < 3; m++) {
         a.W[m] = m < c.n_mats ? c.W[m] : nullptr;
         a.out[m] = m < c.n_mats ? c.out[m] : nullptr;
-        a.n_out[m] = m < c.n_mats ? c.n_out[m] : 0;
-        if (m < c.n_mats && !(c.pair && m > 0)) a.tiles_n += (c.n_out[m] + rows - 1) / rows;
+        a.ld[m] = m < c.n_mats ? c.n_out[m] : 0;
+        const uint32_t here = a.ld[m] > c.row0 ? std::min(a.ld[m] - c.row0, c.rows) : 0;
+        a.n_out[m] = c.row0 + here;
+        if (!(c.pair && m > 0)) a.tiles_n += (here + rows - 1) / rows;
         if (m < 2) a.tile_end[m] = a.tiles_n;
     }
     a.x = c.x;

@@ -137,3 +137,43 @@ def test_millions_of_tokens(dev):
         ia.linear(w.view(torch.uint8).reshape(-1), x, out, ia.linear_desc("F16", n_in, n_out, n_tok, accumulate=acc))
         d = (out - want * (2 if acc else 1)).abs().max()
         assert bool(torch.isfinite(out).all()) and float(d) <= 1e-5 * float(want.abs().max()) * 2
+
+
+@pytest.mark.parametrize("t,n_in,n_out,n_tok", [("F16", 18_000_000, 2, 64), ("Q8_0", 72_000_000, 34, 15), ("F32", 18_000_000, 70, 3)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_rows_beyond_2gib(dev, t, n_in, n_out, n_tok, pair):
+    """Rows so long that a tile's tokens, or a wave's 32 weight rows, span more than 2 GiB. x is zero
+    but for 256 columns (the last among them), so that the sums hold few terms: rel-L2 <= 1e-5 against
+    the same columns in 64 bits, both operands rounded to f16."""
+    import torch
+    import ingot_attn as ia
+
+    g = torch.Generator(device=dev)
+    g.manual_seed(n_out)
+    cols = torch.cat([torch.randint(0, n_in, (255,), generator=g, device=dev), torch.tensor([n_in - 1], device=dev)]).unique()
+    x = torch.zeros(n_tok, n_in, device=dev)
+    x[:, cols] = torch.randn(n_tok, len(cols), generator=g, device=dev)
+
+    def matrix():
+        if t == "Q8_0":
+            raw = torch.randint(0, 256, (n_out, n_in // 32, 34), generator=g, device=dev, dtype=torch.uint8)
+            raw[..., :2] = torch.tensor([0x00, 0x24], dtype=torch.uint8, device=dev)  # d = 2^-6
+            q = raw.view(torch.int8)[:, cols // 32, 2 + cols % 32].double() / 64
+            return raw.reshape(-1), q
+        w = torch.randn(n_out, n_in, generator=g, device=dev)
+        w = w if t == "F32" else w.half()
+        return w.view(torch.uint8).reshape(-1), w[:, cols].half().double()
+
+    xs = x[:, cols].half().double()
+    mats = [matrix() for _ in range(2 if pair else 1)]
+    sums = [xs @ q.t() for _, q in mats]
+    if pair:
+        want = torch.nn.functional.silu(sums[0]) * sums[1]
+        out = torch.empty(n_tok, n_out, device=dev)
+        ia.proj([m for m, _ in mats], x, [out], ia.proj_desc(t, n_in, [n_out, n_out], epilogue=ia.PROJ_SILU_GATE, n_tok=n_tok))
+    else:
+        want = sums[0] * 2
+        out = torch.zeros(n_tok, n_out, device=dev)
+        for _ in range(2):
+            ia.linear(mats[0][0], x, out, ia.linear_desc(t, n_in, n_out, n_tok, accumulate=True), workspace=ia.Workspace(dev))
+    assert float((out - want).norm()) <= 1e-5 * float(want.norm())
