@@ -85,11 +85,6 @@ int launch_rope_kv_store(float* q, const float* k, const float* v, _Float16* k_c
                          uint32_t n_head_kv, uint32_t head_dim, uint32_t pos, uint32_t n_tok,
                          uint32_t q_stride, uint32_t kv_stride, hipStream_t stream);
 
-// Linear layer workspace: split-K completion counters (one 64-byte line per output tile, for up
-// to kLinearMaxTiles tiles), then the partial tiles.
-constexpr size_t kLinearCounterBytes = 16384;
-constexpr uint32_t kLinearMaxTiles = 256;
-
 // out (+)= W·x over a GGUF weight layout (type id as in ggml). With a workspace (zero-filled
 // once) the batched path may split K across workgroups; without one it never does.
 // Returns 0, -1 (grid too large), -2 (type without a kernel) or -4 (launch failed).

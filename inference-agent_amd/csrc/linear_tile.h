@@ -7,7 +7,12 @@
 
 namespace ingot {
 
-// Shape of a call's workgroups: NTB token blocks of 32 per tile (1..5), KG k groups among the
+// Linear layer workspace: split-K completion counters (one 64-byte line per output tile, for up
+// to kLinearMaxTiles tiles), then the partial tiles.
+constexpr size_t kLinearCounterBytes = 16384;
+constexpr uint32_t kLinearMaxTiles = 256;
+
+// Shape of a call's workgroups: NTB token blocks of 32 per tile (1..4), KG k groups among the
 // eight waves (1, 2 or 4: a tile has 256 / KG rows), and the ways n_in is split over workgroups.
 struct TileShape {
     uint32_t ntb, kg, splits;
@@ -35,6 +40,11 @@ constexpr uint32_t tile_cols(uint32_t kg) { return kg == 1 ? 2 : 1; }
 constexpr uint32_t tile_stage(uint32_t kg) { return 64 * kg * tile_cols(kg); }
 // A k group's share of n_in is a multiple of this many elements (whole Q6_K blocks).
 constexpr uint32_t tile_unit(int type) { return type == 14 ? 256 : 64; }
+// n_in in units of every k group's share of that many elements; a call is split over whole units.
+constexpr uint32_t tile_units(int type, uint32_t n_in, uint32_t kg) {
+    const uint64_t u = uint64_t(tile_unit(type)) * kg;
+    return uint32_t((n_in + u - 1) / u);
+}
 // The two x buffers.
 constexpr size_t tile_x_lds(uint32_t ntb, uint32_t kg) { return size_t(2) * 32 * ntb * tile_stage(kg) * 2; }
 // LDS of a workgroup: the x buffers and the waves' weights, reused by the reduction over the k
@@ -46,12 +56,12 @@ constexpr size_t tile_lds(uint32_t ntb, uint32_t kg, size_t w) {
 }
 constexpr size_t tile_bytes(const TileShape& s) { return size_t(tile_rows(s.kg)) * s.ntb * 32 * 4; }
 
-// First token block (32 tokens) of token tile tt: the nb blocks spread evenly over tiles_m tiles, the
-// first nb % tiles_m of them one block longer. (tt * nb / tiles_m would pass 32 bits from 2.1 million
-// tokens of one-block tiles, 4.2 million of four-block tiles on.)
-constexpr uint32_t tile_block0(uint32_t tt, uint32_t nb, uint32_t tiles_m) {
-    const uint32_t longer = nb % tiles_m;
-    return tt * (nb / tiles_m) + (tt < longer ? tt : longer);
+// First of part i's share where n things are spread evenly over `parts`, the first n % parts parts one
+// longer: the token blocks of a token tile, the k units of a split. (i * n / parts would pass 32 bits
+// from 2.1 million tokens of one-block tiles, 4.2 million of four-block tiles on.)
+constexpr uint32_t tile_share0(uint32_t i, uint32_t n, uint32_t parts) {
+    const uint32_t longer = n % parts;
+    return i * (n / parts) + (i < longer ? i : longer);
 }
 
 // 0, -1 (grid too large or a bad shape) or -4 (launch failed). T: the GGUF type id.

@@ -152,7 +152,7 @@ struct TileArgs {
     uint32_t tile_end[2];  // row tiles of matrix m: [tile_end[m-1], tile_end[m])
     const float* x;
     uint32_t n_in, n_tok, row_bytes, accumulate;
-    uint32_t tiles_n, tiles_m, splits, units_per_split, per_xcd;
+    uint32_t tiles_n, tiles_m, splits, units, per_xcd;
     float* part;
     unsigned int* counters;
 };
@@ -185,14 +185,14 @@ void linear_tile_kernel(const TileArgs a) {
     const uint32_t rowbase = a.row0 + rtl * RT + (PAIR ? rg % (RG / 2) : rg) * 32;  // the wave's rows
     // The token blocks are spread evenly over the token tiles.
     const uint32_t nb = (a.n_tok + 31) / 32;
-    const uint32_t tb0 = tile_block0(tt, nb, a.tiles_m), tb1 = tile_block0(tt + 1, nb, a.tiles_m);
+    const uint32_t tb0 = tile_share0(tt, nb, a.tiles_m), tb1 = tile_share0(tt + 1, nb, a.tiles_m);
     const uint32_t tok0 = 32 * tb0, toks = min(a.n_tok - tok0, 32 * (tb1 - tb0));
 
     // This split's elements, in units of KG * unit; each k group takes a contiguous share, U steps
     // of 64 elements a stage.
     constexpr uint32_t unit = tile_unit(T);
-    const uint32_t k0 = split * a.units_per_split * KG * unit;
-    const uint32_t units = min((a.n_in + KG * unit - 1) / (KG * unit) - split * a.units_per_split, a.units_per_split);
+    const uint32_t u0 = tile_share0(split, a.units, a.splits), units = tile_share0(split + 1, a.units, a.splits) - u0;
+    const uint32_t k0 = u0 * KG * unit;
     const uint32_t klen = units * unit, steps = klen / 64, nst = (steps + U - 1) / U;  // per k group
     const bool ragged = k0 + KG * klen > a.n_in || steps % U != 0;  // (elements past the end count as zero)
 
@@ -555,9 +555,9 @@ int launch_tile(const TileCall& c) {
     a.row_bytes = c.n_in / Fmt<T>::blk * Fmt<T>::bytes;
     a.accumulate = c.accumulate;
     a.tiles_m = ((c.n_tok + 31) / 32 + ntb - 1) / ntb;
-    const uint32_t units = (c.n_in + tile_unit(T) * kg - 1) / (tile_unit(T) * kg);
-    a.units_per_split = (units + c.shape.splits - 1) / c.shape.splits;
-    a.splits = (units + a.units_per_split - 1) / a.units_per_split;
+    a.units = tile_units(T, c.n_in, kg);
+    a.splits = c.shape.splits;
+    if (a.splits == 0 || a.splits > std::min(a.units, 8u)) return -1;
     const uint64_t total = uint64_t(a.tiles_n) * a.tiles_m * a.splits, per_xcd = (total + 7) / 8;
     if (per_xcd * 8 > 0x7fffffffu) return -1;
     a.per_xcd = uint32_t(per_xcd);

@@ -26,6 +26,31 @@ def test_every_token_block_once(plan, nb, ntb):
     tiles = -(-nb // ntb)
     pick = range(tiles) if tiles < 70000 else [*range(100), *range(tiles // 2, tiles // 2 + 100), *range(tiles - 100, tiles)]
     for tt in pick:
-        lo, hi = plan.plan_block0(tt, nb, tiles), plan.plan_block0(tt + 1, nb, tiles)
+        lo, hi = plan.plan_share0(tt, nb, tiles), plan.plan_share0(tt + 1, nb, tiles)
         assert 0 < hi - lo <= ntb and lo <= nb and hi <= nb, (tt, lo, hi)
-    assert plan.plan_block0(0, nb, tiles) == 0 and plan.plan_block0(tiles, nb, tiles) == nb
+    assert plan.plan_share0(0, nb, tiles) == 0 and plan.plan_share0(tiles, nb, tiles) == nb
+
+
+def _shape(plan, t, n_in, n_out, n_tok, requested=0, ws=1 << 40):
+    out = (ctypes.c_uint32 * 3)()
+    plan.plan_shape(ctypes.c_uint32(t), ctypes.c_uint32(n_in), ctypes.c_uint32(n_out), ctypes.c_uint32(n_tok),
+                    ctypes.c_uint32(requested), ctypes.c_uint64(ws), out)
+    return tuple(out)  # token blocks, k groups, splits
+
+
+@pytest.mark.parametrize("t", [0, 1, 2, 3, 8, 14, 30])
+def test_splits_are_whole_units(plan, t):
+    """Every chosen split gets at least one unit of n_in (64 elements, 256 of Q6_K, per k group), so
+    that as many splits run as are reported, and a request is met while n_in has 256 elements a split."""
+    unit = 256 if t == 14 else 64
+    for n_in in (256, 512, 1024, 2048, 3072, 5120, 8192, 14336):
+        for n_out in (96, 1024, 3072, 4096, 8192, 14336):
+            for n_tok in (2, 13, 40, 100, 157, 300, 512, 700):
+                for requested in (0, 1, 2, 3, 5, 8):
+                    ntb, kg, splits = _shape(plan, t, n_in, n_out, n_tok, requested)
+                    units = -(-n_in // (unit * kg))
+                    assert 1 <= splits <= units and 1 <= ntb <= 4 and kg in (1, 2, 4)
+                    shares = [plan.plan_share0(i + 1, units, splits) - plan.plan_share0(i, units, splits) for i in range(splits)]
+                    assert sum(shares) == units and min(shares) >= 1
+                    if requested > 1 and -(-n_out // 128) * -(-n_tok // 96) <= 256:  # (counters for 256 tiles)
+                        assert splits == min(requested, max(1, n_in // 256)), (n_in, n_out, n_tok, requested, kg)
