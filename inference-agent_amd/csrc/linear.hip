@@ -898,11 +898,12 @@ int launch_proj(uint32_t type, const void* const* W, const float* x, const float
         if (pro != kProNone || rope) return -2;
         if (epi != kEpiStore && epi != kEpiAccumulate && !pair) return -2;
         if (pair && (n_mats != 2 || n_out[0] != n_out[1])) return -1;
-        for (const bool narrow : {true, false}) {
+        // (the matrices of each number of k groups in one launch: all of them, but for a mix of widths)
+        for (uint32_t kg = 4; kg >= 1; kg /= 2) {
             TileCall c{};
             uint32_t rows = 0;
             for (uint32_t m = 0; m < n_mats; m++) {
-                if ((n_out[m] <= kNarrowRows) != narrow) continue;
+                if (unsplit_k_groups(type, n_in, n_out[m], n_tok) != kg) continue;
                 c.W[c.n_mats] = static_cast<const uint8_t*>(W[m]);
                 c.out[c.n_mats] = pair ? out[0] : out[m];
                 c.n_out[c.n_mats++] = n_out[m];
@@ -914,7 +915,7 @@ int launch_proj(uint32_t type, const void* const* W, const float* x, const float
             c.n_tok = n_tok;
             c.accumulate = epi == kEpiAccumulate;
             c.pair = pair;
-            c.shape = unsplit_shape(type, n_in, rows, n_tok, narrow);
+            c.shape = unsplit_shape(type, n_in, rows, n_tok, kg);
             c.stream = stream;
             const int rc = launch_tile_type(type, c);
             if (rc != 0) return rc;
