@@ -34,8 +34,9 @@
  * groups that are multiples of 3 or 4, as units of 3 or 4 heads) runs
  * the tuned kernel (attn_decode.hip), other head_dim 64/256/128 decode shapes the generic split
  * kernel, prefill at 64/128/256 the MFMA kernel (units of up to 3 heads, 1 at head_dim 256), prefill
- * at every other multiple of 8 below 256 the same kernel with f32 accuracy, and every other
- * head_dim the fallback kernel (attn_naive.hip); the last two never split a prefill. At most 256 query
+ * at every other multiple of 8 below 256 the same kernel with f32 accuracy (but for calls of few
+ * keys and heads, and q rows 2^23 floats apart or more), and everything else the fallback kernel
+ * (attn_naive.hip); the last two never split a prefill. At most 256 query
  * heads (one workspace counter each). Llama-3.2-3B is 24 Q heads / 8 KV heads (group 3);
  * Llama-3.2-1B 32 / 8 with head_dim 64.
  */

@@ -34,7 +34,8 @@ int check_heads(uint32_t n_head, uint32_t n_head_kv, uint32_t head_dim) {
 
 // The head sizes with kernels of their own; every other head_dim up to kMaxHeadDim decodes on the
 // fallback kernel of attn_naive.hip (the reference's naive path, src/metal_backend.mm:373-382) and
-// prefills there or, at a multiple of 8 below 256, on the MFMA kernel (exact_prefill).
+// prefills there or, at a multiple of 8 below 256 and but for the smallest calls, on the MFMA kernel
+// (exact_prefill).
 bool mfma_head_dim(uint32_t hd) { return hd == 64 || hd == 128 || hd == 256; }
 constexpr uint32_t kMaxHeadDim = 1024;
 
@@ -239,8 +240,16 @@ size_t ingot_attn_decode_workspace_size(const IngotAttnDecodeDesc* d) {
 // one, whose 16-byte chunks of a cache row need a multiple of 8, and whose 64 q and out rows of a
 // block lie within the 2 GiB of a descriptor's 32-bit offsets: rows further apart stay on the
 // fallback kernel's 64-bit addresses, as 64-bit ones in the MFMA kernel cost every call 2-7%).
+// Neither do the smallest calls: one 256-key chunk of the fallback kernel in few workgroups (one per
+// head and 8 tokens) ends before the MFMA kernel has staged Q and walked two tiles (8 heads of 96, 33
+// tokens at 150: 8.4 us and 10.5; 24 heads of 192, 2 at 100: 8.4 and 12.0; with 120 workgroups the
+// two meet near 100 keys, 24 heads of 96, 33 at 60: 9.0 and 8.7). Heads below 64 walk shorter tiles and
+// win from 64 workgroups on, those below 24 always (padded to 64, but with little else to do).
 bool exact_prefill(const IngotAttnPrefillDesc* d) {
-    return d->head_dim % 8 == 0 && d->head_dim < 256 && d->q_stride <= 0x7fffffffu / (64 * sizeof(float));
+    if (d->head_dim % 8 != 0 || d->head_dim >= 256 || d->q_stride > 0x7fffffffu / (64 * sizeof(float))) return false;
+    const uint64_t keys = uint64_t(d->pos) + d->n_tok, wgs = (uint64_t(d->n_tok) + 7) / 8 * d->n_head;
+    const bool small = keys <= 256 && wgs <= (d->head_dim < 64 ? 64 : 128) && wgs * keys <= 16384;
+    return !small || d->head_dim < 24;
 }
 
 size_t ingot_attn_prefill_workspace_size(const IngotAttnPrefillDesc* d) {

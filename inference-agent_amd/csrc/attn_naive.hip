@@ -1,5 +1,6 @@
 // attn_naive.hip — attention for head sizes the MFMA kernels do not cover: decode for anything but
-// 64, 128 and 256, causal prefill where the head size is no multiple of 8 or above 256; up to 1024.
+// 64, 128 and 256, causal prefill where the head size is no multiple of 8 or above 256, and the
+// smallest prefills of the other sizes; up to 1024.
 //
 // The counterpart of the reference's naive `attention` kernel (shaders/kernels.metal:639-702),
 // which src/metal_backend.mm:373-382 runs for every shape outside its flash paths: query i of

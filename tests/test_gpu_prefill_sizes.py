@@ -28,7 +28,13 @@ def dev():
 
 @pytest.mark.parametrize("hd,nh,nkv,pos,n,pad", [
     (8, 2, 1, 0, 2, 0), (56, 4, 2, 31, 33, 0), (72, 3, 1, 63, 65, 3), (96, 6, 2, 127, 64, 0),
-    (120, 2, 2, 190, 129, 1), (136, 4, 1, 5, 70, 0), (248, 2, 1, 33, 31, 2)])
+    (120, 2, 2, 190, 129, 1), (136, 4, 1, 5, 70, 0), (248, 2, 1, 33, 31, 2),
+    # (calls of one key chunk and few workgroups run the fallback kernel: the same sizes with more keys)
+    (24, 2, 2, 255, 2, 0), (56, 4, 2, 261, 33, 0), (72, 3, 1, 263, 65, 3), (96, 6, 2, 327, 64, 0), (136, 4, 1, 205, 70, 0),
+    (248, 2, 1, 233, 31, 2), (200, 2, 1, 1000, 5, 4),
+    # and both sides of that line
+    (96, 8, 8, 0, 128, 0), (96, 8, 8, 1, 128, 0), (96, 8, 8, 192, 64, 0), (96, 8, 8, 193, 64, 0), (40, 8, 2, 100, 64, 0),
+    (40, 8, 2, 100, 65, 0), (96, 17, 17, 0, 64, 0)])
 @pytest.mark.parametrize("gain,bar", [(1.0, 2e-6), (100.0, 2e-5)])
 def test_zero_filled_dims(dev, hd, nh, nkv, pos, n, pad, gain, bar):
     import torch
@@ -64,7 +70,7 @@ def test_rows_beyond_2gib(dev):
     import torch
     import ingot_attn as ia
 
-    hd, nh, nkv, pos, n = 96, 3, 1, 40, 64
+    hd, nh, nkv, pos, n = 96, 3, 1, 400, 64
     g = torch.Generator(device=dev)
     g.manual_seed(1)
     q = torch.randn(n, nh * hd, generator=g, device=dev)
@@ -127,16 +133,16 @@ def test_any_finite_query(dev, hd, size):
     import torch
     import ingot_attn as ia
 
-    n = 40
+    n, pos = 40, 300
     rng = np.random.default_rng(hd)
-    k = rng.standard_normal((n, hd)).astype(np.float16)
-    v = rng.standard_normal((n, hd)).astype(np.float16)
+    k = rng.standard_normal((pos + n, hd)).astype(np.float16)
+    v = rng.standard_normal((pos + n, hd)).astype(np.float16)
     q = (rng.standard_normal((n, hd)) * size).astype(np.float32)
     t = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
     out = torch.empty(n, hd, device=dev)
-    ia.attn_prefill(t(q), t(k), t(v), out, ia.prefill_desc(1, 1, hd, 0, n))
+    ia.attn_prefill(t(q), t(k), t(v), out, ia.prefill_desc(1, 1, hd, pos, n))
     s = q.astype(np.float64) @ k.astype(np.float64).T / np.sqrt(hd)
-    s[np.arange(n)[None, :] > np.arange(n)[:, None]] = -np.inf
+    s[np.arange(pos + n)[None, :] > pos + np.arange(n)[:, None]] = -np.inf
     p = np.exp(s - s.max(1, keepdims=True))
     want = p / p.sum(1, keepdims=True) @ v.astype(np.float64)
     got = out.cpu().numpy()
