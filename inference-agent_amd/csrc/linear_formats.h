@@ -68,13 +68,12 @@ __device__ __forceinline__ uint32_t col_offset(uint32_t c) {
     else return c * Col<T>::bytes;
 }
 
-// The window of the column at byte offset off + soff (relative to a 16-byte aligned buffer base;
-// soff wave-uniform, a multiple of 4, not for Q6_K).
+// The window of the column at byte offset off (relative to a 16-byte aligned buffer base).
 template <int T>
 __device__ __forceinline__ void col_load(const __amdgpu_buffer_rsrc_t& rs, uint32_t off, uint32_t (&w)[Col<T>::ndw],
-                                         uint32_t c = 0, uint32_t soff = 0) {
+                                         uint32_t c = 0) {
     auto ld4 = [&](uint32_t o, int at) {
-        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, int(o), int(soff), 0));
+        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, int(o), 0, 0));
         w[at] = v[0]; w[at + 1] = v[1]; w[at + 2] = v[2]; w[at + 3] = v[3];
     };
     if constexpr (T == kQ6_K) {
@@ -90,13 +89,11 @@ __device__ __forceinline__ void col_load(const __amdgpu_buffer_rsrc_t& rs, uint3
         w[19] = __builtin_amdgcn_raw_buffer_load_b32(rs, int((off + 208) & ~3u), 0, 0);
     } else if constexpr (T == kF16 || T == kBF16) {
         for (int i = 0; i < 4; i++) ld4(off + 16 * i, 4 * i);
-    } else if constexpr (T == kF32) {
-        for (int i = 0; i < 8; i++) ld4(off + 16 * i, 4 * i);
     } else {
         const uint32_t p = off & ~3u;
         ld4(p, 0);
         if constexpr (T == kQ8_0) ld4(p + 16, 4);
-        w[Col<T>::ndw - 1] = __builtin_amdgcn_raw_buffer_load_b32(rs, int(p + 4 * (Col<T>::ndw - 1)), int(soff), 0);
+        w[Col<T>::ndw - 1] = __builtin_amdgcn_raw_buffer_load_b32(rs, int(p + 4 * (Col<T>::ndw - 1)), 0, 0);
     }
 }
 

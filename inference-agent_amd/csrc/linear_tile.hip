@@ -249,8 +249,8 @@ void linear_tile_kernel(const TileArgs a) {
     static_assert(BM % RPP == 0, "x staging");
     typedef _Float16 half4_ __attribute__((ext_vector_type(4)));
     // (16-byte chunks are XOR-swizzled by the row so that 16 rows' reads of one chunk cover the 64
-    // banks: a 128-byte row spans half of them, a longer one all)
-    auto xswz = [](uint32_t r) { return SK == 64 ? (r >> 1) & 7 : r & 15; };
+    // banks: a row spans all of them)
+    auto xswz = [](uint32_t r) { return r & 15; };
     const uint32_t tr = tid / FPR, tc = tid % FPR;
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(a.x + size_t(tok0) * a.n_in), 0, int(4 * toks * a.n_in), kBufferFlags);
@@ -565,14 +565,15 @@ int launch_tile(const TileCall& c) {
     a.part = a.splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(c.workspace) + kLinearCounterBytes) : nullptr;
     const dim3 grid(uint32_t(per_xcd * 8));
     switch (kg * 8 + ntb) {
-#define INGOT_SHAPE(KGv, NTBv) \
-    case KGv * 8 + NTBv:       \
-        return c.pair ? launch<T, NTBv, KGv, true>(a, grid, c.stream) : launch<T, NTBv, KGv, false>(a, grid, c.stream)
+// (the shapes without a kernel: tile_cost of linear_shape.h)
+#define INGOT_SHAPE(KGv, NTBv)                                         \
+    case KGv * 8 + NTBv:                                               \
+        if constexpr (T != kF32 || (NTBv < 4 && KGv * NTBv != 12))     \
+            return c.pair ? launch<T, NTBv, KGv, true>(a, grid, c.stream) : launch<T, NTBv, KGv, false>(a, grid, c.stream); \
+        else return -1
         INGOT_SHAPE(4, 1);
         INGOT_SHAPE(4, 2);
-        case 4 * 8 + 3:
-            if constexpr (T != kF32) return c.pair ? launch<T, 3, 4, true>(a, grid, c.stream) : launch<T, 3, 4, false>(a, grid, c.stream);
-            else return -1;
+        INGOT_SHAPE(4, 3);
         INGOT_SHAPE(2, 2);
         INGOT_SHAPE(2, 3);
         INGOT_SHAPE(2, 4);

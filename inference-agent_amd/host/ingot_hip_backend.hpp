@@ -60,12 +60,13 @@ struct HostModel {
 class HipBackend {
 public:
     // Tiles (256 rows x 64 tokens, over q, k and v) from which a chunk's q/k/v run as one batched
-    // launch instead of three split-K launches: every chunk (Llama-3.2-3B Q4_0: 13 tokens 12.9 us
-    // against 25, 157 tokens 24.1 against 33.8, 512 tokens 34.8 against 56.7).
+    // launch instead of three split-K launches: every chunk (Llama-3.2-3B Q4_0: 13 tokens 13.7 us
+    // against 24.6, 157 tokens 20.9 against 34.1, 512 tokens 33.9 against 77.0). A number above a
+    // chunk's tiles forces the three launches.
     uint32_t qkv_one_launch_min_tiles = 0;
     // Tiles (128 rows of gate and of up x 64 tokens) from which a chunk's gate/up + silu run as
-    // one batched launch: every chunk (Llama-3.2-3B Q4_0: 13 tokens 18.1 us against 25.1 and the
-    // silu launch, 157 tokens 36.7 against 49.3).
+    // one batched launch: every chunk (Llama-3.2-3B Q4_0, against two and the silu launch: 13 tokens
+    // 18.6 us against 26.2, 157 tokens 36.5 against 51.7, 512 tokens 65.3 against 95.8).
     uint32_t ffn_one_launch_min_tiles = 0;
 
     // device_weights: the matrices' `data` are device addresses already (gguf::DeviceWeights);

@@ -22,8 +22,9 @@ import ingot_attn as ia
 
 
 # Tiles (256 rows x 64 tokens over q, k and v) from which a chunk's q/k/v run as one batched
-# launch: every chunk (Llama-3.2-3B Q4_0: 13 tokens 12.9 us in one launch, 25 in three; 157 tokens
-# 24.1 and 33.8; 512 tokens 34.8 and 56.7). A number above a chunk's tiles forces the three launches.
+# launch: every chunk (Llama-3.2-3B Q4_0: 13 tokens 13.7 us in one launch, 24.6 in three; 157 tokens
+# 20.9 and 34.1; 512 tokens 33.9 and 77.0; the three were faster only at 40 to 160 tokens of 8192-wide
+# q with 1024-wide k and v, by 11 to 22%). A number above a chunk's tiles forces the three launches.
 QKV_ONE_LAUNCH_MIN_TILES = 0
 
 
@@ -35,8 +36,9 @@ def qkv_one_launch(n_tok, q_dim, kv_dim):
 
 
 # Tiles (128 rows of gate and of up x 64 tokens) from which a chunk's gate/up + silu run as one
-# batched launch: every chunk (Llama-3.2-3B Q4_0: 13 tokens 18.1 us in one launch, 25.1 in two before
-# ingot_silu_mul; 157 tokens 36.7 and 49.3).
+# batched launch: every chunk (Llama-3.2-3B Q4_0, with ingot_silu_mul after the two: 13 tokens 18.6
+# us in one launch, 26.2 in two; 157 tokens 36.5 and 51.7; 512 tokens 65.3 and 95.8). A number above a
+# chunk's tiles forces the two launches.
 FFN_ONE_LAUNCH_MIN_TILES = 0
 
 

@@ -109,7 +109,10 @@ int main() {
             const int32_t bad[2] = {1, m.n_vocab};
             expect(throws([&] { b.forward_batch(bad, 2, 0); }, "token id out of range"), "token id error");
         }
-        {   // wq, wk, wv of one type and the one-launch q/k/v path forced: a chunk, then decode steps
+        // wq, wk, wv of one type: a chunk with q/k/v and gate/up in one launch each (the default) and in
+        // separate ones (a threshold that no chunk reaches), then decode steps
+        for (const uint32_t min_tiles : {0u, 1u << 30}) {
+            const char* const how = min_tiles ? "separate" : "one-launch";
             synth::Owned own2;
             const ingot::HostModel m2 = synth::make_model(own2, 12, true);
             std::vector<OracleLayer> ol2;
@@ -124,21 +127,21 @@ int main() {
             std::fill(kc.begin(), kc.end(), 0);
             std::fill(vc.begin(), vc.end(), 0);
             ingot::HipBackend b(m2, n_ctx, 48);
-            b.qkv_one_launch_min_tiles = 0;
-            b.ffn_one_launch_min_tiles = 0;
+            b.qkv_one_launch_min_tiles = min_tiles;
+            b.ffn_one_launch_min_tiles = min_tiles;
             const int n = 40;
             const float* got = b.forward_batch(toks.data(), n, 0);
             for (int p = 0; p < n; p++)
                 oracle_forward(&om2, kc.data(), vc.data(), n_ctx, toks[size_t(p)], p, want.data(), 1, 8);
             double r = rel_l2(got, want.data(), m2.n_vocab);
             char buf[96];
-            std::snprintf(buf, sizeof buf, "one-launch q/k/v and gate/up prefill 40 tokens: rel-L2 %.3e", r);
+            std::snprintf(buf, sizeof buf, "%s q/k/v and gate/up prefill 40 tokens: rel-L2 %.3e", how, r);
             expect(r <= 5e-3, buf);
             for (int p = n; p < n + 3; p++) {
                 got = b.forward(toks[size_t(p)], p);
                 oracle_forward(&om2, kc.data(), vc.data(), n_ctx, toks[size_t(p)], p, want.data(), 0, 8);
                 r = rel_l2(got, want.data(), m2.n_vocab);
-                std::snprintf(buf, sizeof buf, "one-launch q/k/v, decode pos %d: rel-L2 %.3e", p, r);
+                std::snprintf(buf, sizeof buf, "%s q/k/v, decode pos %d: rel-L2 %.3e", how, p, r);
                 expect(r <= 5e-3, buf);
             }
         }

@@ -154,9 +154,9 @@ def test_forward_prefill_then_decode(dev, oracle_mod, types, prefill):
 @pytest.mark.parametrize("types", ["F16", "Q4_0"])
 @pytest.mark.parametrize("which", ["qkv", "ffn", "both"])
 def test_forward_prefill_one_launch_qkv(dev, oracle_mod, monkeypatch, types, which):
-    """The chunk's q/k/v through one batched ingot_proj launch, and/or its gate/up + silu
-    through one (forced; the real thresholds need a Llama-3.2-3B-sized chunk): logits, the K
-    cache rows it wrote and the decode steps after it against the oracle forward."""
+    """The chunk's q/k/v through one batched ingot_proj launch, and its gate/up + silu through one
+    (the default): logits, the K cache rows it wrote and the decode steps after it against the oracle
+    forward."""
     import ingot_forward
 
     if which in ("qkv", "both"):
@@ -170,6 +170,33 @@ def test_forward_prefill_one_launch_qkv(dev, oracle_mod, monkeypatch, types, whi
     a = kc_gpu.view(np.float16).astype(np.float64)
     b = kc_orc.view(np.float16).astype(np.float64)
     assert np.linalg.norm(a - b) / np.linalg.norm(b) <= 1e-2
+
+
+@pytest.mark.parametrize("types", ["F16", "Q4_0"])
+@pytest.mark.parametrize("which", ["qkv", "ffn", "both"])
+def test_forward_prefill_separate_launches(dev, oracle_mod, monkeypatch, types, which):
+    """The chunk's q/k/v through three ingot_linear calls, and/or its gate/up through two and
+    ingot_silu_mul (forced by a threshold that no chunk reaches; weights of one type): against the
+    oracle forward, and against the one-launch forward, from which it differs by the order of f32 sums
+    (and what f16 roundings of the next products' inputs make of it)."""
+    import ingot_forward
+
+    one, kc_one, _ = _run(dev, oracle_mod, types, prefill=45, decode_steps=3, tied=True)
+    if which in ("qkv", "both"):
+        monkeypatch.setattr(ingot_forward, "QKV_ONE_LAUNCH_MIN_TILES", 1 << 30)
+    if which in ("ffn", "both"):
+        monkeypatch.setattr(ingot_forward, "FFN_ONE_LAUNCH_MIN_TILES", 1 << 30)
+    calls = []
+    monkeypatch.setattr(ingot_forward.ia, "proj", lambda *a, _p=ingot_forward.ia.proj, **k: (calls.append(a[3].n_tok), _p(*a, **k)))
+    res, kc_gpu, kc_orc = _run(dev, oracle_mod, types, prefill=45, decode_steps=3, tied=True)
+    assert calls.count(45) == {"qkv": 1, "ffn": 1, "both": 0}[which] * CFG["n_layer"]  # batched one-launch calls left
+    for (what, g, w), (_, g1, _) in zip(res, one):
+        assert np.all(np.isfinite(g))
+        assert _rel(g, w) <= 5e-3, (what, _rel(g, w))
+        assert _rel(g, g1) <= 1e-3, (what, _rel(g, g1))
+    a, b, c = (k.view(np.float16).astype(np.float64) for k in (kc_gpu, kc_orc, kc_one))
+    assert np.linalg.norm(a - b) / np.linalg.norm(b) <= 1e-2
+    assert np.linalg.norm(a - c) / np.linalg.norm(c) <= 1e-3
 
 
 @pytest.mark.parametrize("head_dim,n_head,n_head_kv", [(64, 8, 2), (256, 4, 2), (128, 8, 1)])
