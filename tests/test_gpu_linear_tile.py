@@ -71,9 +71,10 @@ def test_ragged_end_reads_no_neighbour(dev, t):
 
 @pytest.mark.parametrize("t", ["Q4_0", "F16"])
 @pytest.mark.parametrize("n_tok", [40, 130, 300])
-def test_chunk_of_narrow_and_wide_matrices(dev, t, n_tok):
-    """Matrices on both sides of the 4096 rows where the number of k groups changes, in one
-    ingot_proj call: each output equals ingot_linear (n_splits = 1) on its matrix bit for bit."""
+def test_chunk_of_narrow_and_wide_matrices(dev, oracle_mod, t, n_tok):
+    """Matrices narrower and wider than n_in, which take different numbers of k groups, in one
+    ingot_proj call: each output equals ingot_linear (n_splits = 1) on its matrix bit for bit, and the
+    oracle within the bar."""
     import torch
     import ingot_attn as ia
 
@@ -81,15 +82,19 @@ def test_chunk_of_narrow_and_wide_matrices(dev, t, n_tok):
     g = torch.Generator(device=dev)
     g.manual_seed(n_tok)
     x = torch.randn(n_tok, n_in, generator=g, device=dev)
-    ws = [torch.from_numpy(gb.random_weights(t, n, n_in, seed=n).reshape(-1)).to(dev) for n in n_outs]
+    raw = [gb.random_weights(t, n, n_in, seed=n) for n in n_outs]
+    ws = [torch.from_numpy(w.reshape(-1)).to(dev) for w in raw]
     outs = [torch.zeros(n_tok, n, device=dev) for n in n_outs]
     refs = [torch.zeros(n_tok, n, device=dev) for n in n_outs]
     ia.proj(ws, x, outs, ia.proj_desc(t, n_in, list(n_outs), n_tok=n_tok))
     for w, r, n in zip(ws, refs, n_outs):
         ia.linear(w, x, r, ia.linear_desc(t, n_in, n, n_tok, n_splits=1), use_workspace=False)
     torch.cuda.synchronize()
-    for o, r in zip(outs, refs):
+    for o, r, w, n in zip(outs, refs, raw, n_outs):
         assert torch.equal(o, r) and bool(torch.isfinite(o).all())
+        want = oracle_mod.linear(t, w, x.cpu().numpy(), n_in, n, f16_path=True)
+        d = np.abs(o.cpu().numpy() - want)
+        assert d.max() <= 1e-5 * np.abs(want).max() + 1e-6 and np.linalg.norm(d) <= 1e-5 * np.linalg.norm(want)
 
 
 @pytest.mark.parametrize("t", ["Q4_0", "Q4_1", "Q8_0", "Q6_K"])
