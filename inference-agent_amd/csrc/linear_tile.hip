@@ -23,6 +23,7 @@
 // interleaving MFMAs with it (67 M wave-cycles, 52 M without); starting the token tiles at
 // different stages, as the L2 channels would like it, changed nothing.
 #include <algorithm>
+#include <type_traits>
 
 #include "linear_formats.h"
 #include "linear_tile.h"
@@ -121,6 +122,14 @@ template <> struct WStage<kQ4_0> { static constexpr uint32_t WK = 256, CH = 10, 
 template <> struct WStage<kQ4_1> { static constexpr uint32_t WK = 256, CH = 12, pitch = 208; };
 template <> struct WStage<kQ6_K> { static constexpr uint32_t WK = 256, CH = 14, pitch = 240; };
 
+// On one k group the 16-bit types take stages of 128 elements, whole 256-byte pieces of a row, which
+// come faster from HBM (F16 and BF16 weights that no cache holds, mean of 19 token counts by 10 sets of
+// matrices: 1.05 to 1.08x); on more, where a wave's share is short, the longer first load costs more
+// (0.91 to 0.99x).
+struct WStage128 { static constexpr uint32_t WK = 128, CH = 16, pitch = 272; };
+template <int T, int KG>
+using Staged = std::conditional_t<KG == 1 && (T == kF16 || T == kBF16), WStage128, WStage<T>>;
+
 // The window of the column at byte `off` of a row in LDS (col_load's dwords).
 template <int T>
 __device__ __forceinline__ void col_read(const uint8_t* row, uint32_t off, uint32_t c, uint32_t (&w)[Col<T>::ndw]) {
@@ -202,7 +211,7 @@ void linear_tile_kernel(const TileArgs a) {
     const uint64_t left = (uint64_t(n_out) * a.row_bytes - wbase + 15) & ~uint64_t(15);
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t*>(W + wbase), 0, int(left < 0x7ffffff0u ? left : 0x7ffffff0u), kBufferFlags);
-    using WS = WStage<T>;
+    using WS = Staged<T, KG>;
     constexpr uint32_t WSB = WS::WK / Fmt<T>::blk * Fmt<T>::bytes, NCH = 32 * WS::CH / 64, QS = WS::WK / 64;
     static_assert(32 * WS::CH % 64 == 0 && WS::CH * 16 <= WS::pitch, "whole rounds of chunks");
     uint8_t* const wsm = smem + tile_x_lds(NTB, KG) + wave * (32 * WS::pitch);
@@ -493,7 +502,7 @@ void linear_tile_kernel(const TileArgs a) {
 
 template <int T, int NTB, int KG, bool PAIR>
 int launch(const TileArgs& a, dim3 grid, hipStream_t stream) {
-    constexpr size_t lds = tile_lds(NTB, KG, 256 * WStage<T>::pitch);
+    constexpr size_t lds = tile_lds(NTB, KG, 256 * Staged<T, KG>::pitch);
     static_assert(lds + 16 <= 160 * 1024, "LDS");
     static const hipError_t attr = hipFuncSetAttribute(
         reinterpret_cast<const void*>(&linear_tile_kernel<T, NTB, KG, PAIR>),
