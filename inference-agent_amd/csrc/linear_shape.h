@@ -19,13 +19,13 @@ struct TileCost {
     float row256;
 };
 inline const TileCost& tile_cost(uint32_t type) {
-    static constexpr TileCost q4_0{{{0, 2.4f, 3.7f, 5.1f, 0}, {0, 0, 6.1f, 7.4f, 9.1f}, {0, 0, 9.7f, 11.4f, 13.3f}}, 144};
-    static constexpr TileCost q4_1{{{0, 3.3f, 4.5f, 5.7f, 0}, {0, 0, 7.5f, 8.8f, 10.1f}, {0, 0, 12.2f, 13.9f, 15.6f}}, 160};
-    static constexpr TileCost q8_0{{{0, 3.3f, 4.9f, 6.1f, 0}, {0, 0, 7.4f, 9.2f, 11.2f}, {0, 0, 12.6f, 14.1f, 16.1f}}, 272};
-    static constexpr TileCost q6_k{{{0, 5.0f, 6.3f, 8.6f, 0}, {0, 0, 10.8f, 11.5f, 14.3f}, {0, 0, 17.5f, 19.3f, 24.1f}}, 210};
-    static constexpr TileCost f16{{{0, 2.2f, 3.6f, 5.2f, 0}, {0, 0, 5.3f, 6.9f, 9.0f}, {0, 0, 9.3f, 11.5f, 14.1f}}, 512};
-    static constexpr TileCost bf16{{{0, 2.4f, 4.0f, 5.5f, 0}, {0, 0, 5.9f, 7.5f, 9.5f}, {0, 0, 10.1f, 11.6f, 14.5f}}, 512};
-    static constexpr TileCost f32{{{0, 4.2f, 5.9f, 0, 0}, {0, 0, 9.1f, 11.0f, 0}, {0, 0, 16.0f, 18.6f, 0}}, 1024};
+    static constexpr TileCost q4_0{{{0, 2.8f, 4.2f, 5.7f, 0}, {0, 0, 6.7f, 8.0f, 9.8f}, {0, 0, 10.1f, 11.7f, 13.5f}}, 144};
+    static constexpr TileCost q4_1{{{0, 3.7f, 5.0f, 6.4f, 0}, {0, 0, 8.2f, 9.5f, 10.9f}, {0, 0, 12.7f, 14.4f, 16.1f}}, 160};
+    static constexpr TileCost q8_0{{{0, 3.8f, 5.6f, 7.0f, 0}, {0, 0, 8.3f, 10.1f, 12.2f}, {0, 0, 13.1f, 14.8f, 16.5f}}, 272};
+    static constexpr TileCost q6_k{{{0, 5.5f, 6.8f, 9.3f, 0}, {0, 0, 11.5f, 12.3f, 15.2f}, {0, 0, 17.9f, 19.8f, 25.0f}}, 210};
+    static constexpr TileCost f16{{{0, 3.5f, 5.3f, 7.2f, 0}, {0, 0, 7.5f, 9.3f, 11.4f}, {0, 0, 11.6f, 13.8f, 15.5f}}, 512};
+    static constexpr TileCost bf16{{{0, 3.7f, 5.7f, 7.5f, 0}, {0, 0, 8.0f, 10.0f, 12.1f}, {0, 0, 12.4f, 14.6f, 16.0f}}, 512};
+    static constexpr TileCost f32{{{0, 5.1f, 7.0f, 0, 0}, {0, 0, 10.6f, 12.6f, 0}, {0, 0, 18.2f, 20.8f, 0}}, 1024};
     switch (type) {
         case 0:  return f32;
         case 1:  return f16;
@@ -51,13 +51,13 @@ inline uint64_t tile_count(uint32_t n_out, uint32_t n_tok, const TileShape& s) {
 
 // Estimated time (us) of a shape on n_out rows: the launch; rounds of 256 workgroups, each a fixed part
 // and the longest share of n_in (whole units), slower the more W and x the workgroups read from the
-// L2s, and hardly faster than the eight XCDs fetch their shares of x (5.7 TB/s) and W (4.7 TB/s);
+// L2s, and hardly faster than the eight XCDs fetch their shares of x (6.2 TB/s) and W (3.6 TB/s);
 // the output's stores; and where n_in is split the partial tiles' stores and the last workgroup's
-// reading them. Fitted to 59 thousand timings: seven types, 24 sets of matrices (512 .. 14336
-// columns, 512 .. 28672 rows), 2 to 1024 tokens, every shape (rms 8%). Against the best shape timed, the
-// one it picks is 0.7% slower in the mean and 4% in the worst twentieth (one matrix; 0.1% and 0 q/k/v,
-// 0.3% and 1.6% gate/up). One table in proportion for all types was 3 to 7% off in the mean, F16 3072 x
-// 3072 at 512 tokens 32.5 us for 26.7.
+// reading them. Fitted to 133 thousand timings, over half with weights that no cache holds, as a
+// model's are: seven types, 24 sets of matrices (512 .. 14336 columns, 512 .. 28672 rows), 2 to 1024
+// tokens, every shape. Against the best shape timed, the one it picks is 0.8% slower in the mean and 5%
+// in the worst twentieth (one matrix; 0.1% and 0 q/k/v, 0.4% and 4% gate/up). The former rule, one
+// table in proportion for all types, took 2.4% more over single matrices and 5 to 6% over sets.
 inline float tile_us(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_tok, const TileShape& s) {
     const TileCost& c = tile_cost(type);
     const uint32_t tiles_m = ((n_tok + 31) / 32 + s.ntb - 1) / s.ntb, rows = tile_rows(s.kg);
@@ -66,16 +66,16 @@ inline float tile_us(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_to
     const uint32_t share = (tile_units(type, n_in, s.kg) + s.splits - 1) / s.splits * tile_unit(type) * s.kg;
     const float k = float(share) / 1024.f, row = c.row256 / 256.f;
     const float reads = (float(rows) * row + 128.f * float(s.ntb)) / 256.f;  // of an element of n_in, 256 bytes
-    const float walk = rounds * (3.2f + k * c.walk[tile_kg_row(s.kg)][s.ntb]) + 0.8f * k * reads * wgs / 256.f;
+    const float walk = rounds * (2.8f + k * c.walk[tile_kg_row(s.kg)][s.ntb]) + 0.4f * k * reads * wgs / 256.f;
     // An XCD takes a contiguous run of (row tile, token tile, split) ids: the part of x and of W in it.
     const float run = float(uint64_t(wgs + 7.f) / 8), turns = run / (float(tiles_m) * splits);
     const float x = std::min(1.f, turns) * float(n_tok) * 4.f;
     const float w = (run >= splits ? std::max(1.f, turns) : run / splits) * float(rows) * row;
-    const float fetch = 8e-7f * float(n_in) * (1.4f * x + 1.7f * w);
+    const float fetch = 8e-7f * float(n_in) * (1.3f * x + 2.2f * w);
     const float w2 = walk * walk, f2 = fetch * fetch, part = float(tile_bytes(s));
-    const float t = 2.4f + std::sqrt(std::sqrt(w2 * w2 + f2 * f2)) + 2.1e-7f * wgs * part;
+    const float t = 2.9f + std::sqrt(std::sqrt(w2 * w2 + f2 * f2)) + 2.5e-7f * wgs * part;
     if (s.splits == 1) return t;
-    return t + 0.9f + 0.3f * splits * part / 32768.f + 1e-7f * wgs * part;
+    return t + 1.f + 0.3f * splits * part / 32768.f + 6e-8f * wgs * part;
 }
 
 // The tile height of least estimated time; it does not change the order of an output's sum.
@@ -144,7 +144,7 @@ inline TileShape linear_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint
                 const uint64_t tiles = tile_count(n_out, n_tok, s);
                 if (splits > 1 && (tiles > kLinearMaxTiles ||
                                    kLinearCounterBytes + tiles * splits * tile_bytes(s) > workspace_bytes)) continue;
-                const float u = tile_us(type, n_in, n_out, n_tok, s) * (splits == 1 ? 1.f : n_tok <= 128 ? 0.98f : 1.02f);
+                const float u = tile_us(type, n_in, n_out, n_tok, s) * (splits == 1 ? 1.f : n_tok <= 128 ? 0.98f : 1.03f);
                 if (best.ntb == 0 || u < t) { best = s; t = u; }
             }
     }
