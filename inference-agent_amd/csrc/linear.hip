@@ -745,11 +745,11 @@ int launch_stream_t(MvArgs a, uint32_t n_mats, int pro, int epi, hipStream_t str
         if (count(256, r, false) >= 256 || r == min_rph) { nt = 256; rph = r; }
     if (!nt) { nt = 256; rph = min_rph; }  // (Q6_K pairs: min_rph above kMaxRph)
     a.blocks = count(nt, rph, true);
-    // A block-quantized call of more row blocks than the chip holds workgroups (a vocabulary) loops
-    // over them: staging and normalizing x otherwise costs each workgroup as much as its rows.
-    // Logits of 128256 x 3072 (rmsnorm), 16032 / 4008 blocks on 2048 workgroups: Q6_K 101.0 -> 82.9
-    // us, Q4_0 56.0 -> 47.3, Q8_0 90.8 -> 80.1 (1024: 86.1, 48.3, 79.7; 512: 95.8, 49.1, 82.5); F16
-    // rows gain nothing (134.5, 136.0).
+    // A block-quantized call of many more row blocks than the chip holds workgroups (a vocabulary; six
+    // of 24 KB fit a CU, 1536 in all) loops over them: staging and normalizing x otherwise costs each
+    // workgroup as much as its rows. Logits of 128256 x 3072 (rmsnorm), 16032 / 4008 blocks on 2048
+    // workgroups: Q6_K 101.0 -> 82.9 us, Q4_0 56.0 -> 47.3, Q8_0 90.8 -> 80.1 (1024: 86.1, 48.3, 79.7;
+    // 512: 95.8, 49.1, 82.5); F16 rows gain nothing (134.5, 136.0).
     constexpr uint32_t kLoopGrid = 2048;
     uint32_t blocks = a.blocks;
     if (Fmt<T>::blk > 1 && nt == 256 && epi == kEpiStore && blocks > kLoopGrid) {

@@ -123,8 +123,10 @@ inline TileShape unsplit_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uin
 // The shape of a call on one matrix whose workspace lets n_in be split: of all shapes, the one of
 // least estimated time (wo 3072 x 3072 Q4_0 at 13 tokens: 13.1 us unsplit, 9.1 in five; down
 // 8192 x 3072 at 157: 64.8 and 27.5 us); a split costs up to 2% less than estimated up to 128 tokens
-// (Q4_0 3072 x 3072 at 128: 14.2 us in two, 14.5 unsplit) and more beyond. A requested count takes two k groups, or one where n_in has
-// too few units of two.
+// (Q4_0 3072 x 3072 at 128: 14.2 us in two, 14.5 unsplit) and more beyond, where the last workgroup of a
+// large tile also adds to out (wo at 512: 30.8 unsplit, 31.9 in two; of 1862 such calls 33 were more than
+// 3% slower than the former rule's choice with 1.06 here, 42 with 1.03). A requested count takes two
+// k groups, or one where n_in has too few units of two.
 inline TileShape linear_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_tok, uint32_t requested,
                               size_t workspace_bytes) {
     const uint32_t cap = std::min(kMaxSplits, std::max(1u, n_in / 256));  // at least 256 elements a split
@@ -144,7 +146,7 @@ inline TileShape linear_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint
                 const uint64_t tiles = tile_count(n_out, n_tok, s);
                 if (splits > 1 && (tiles > kLinearMaxTiles ||
                                    kLinearCounterBytes + tiles * splits * tile_bytes(s) > workspace_bytes)) continue;
-                const float u = tile_us(type, n_in, n_out, n_tok, s) * (splits == 1 ? 1.f : n_tok <= 128 ? 0.98f : 1.03f);
+                const float u = tile_us(type, n_in, n_out, n_tok, s) * (splits == 1 ? 1.f : n_tok <= 128 ? 0.98f : 1.06f);
                 if (best.ntb == 0 || u < t) { best = s; t = u; }
             }
     }
