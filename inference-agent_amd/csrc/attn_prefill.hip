@@ -88,6 +88,46 @@ template <int HD> __device__ __forceinline__ int swz_v(int row) {
     return HD == 64 ? ((row >> 1) & 3) << 1 : (row & 7) << 1;
 }
 
+// One query of a head over keys [0, n_keys) in f32, by one wave: a lane per key for the scores, a lane
+// per HD / 64 dims for the sums. What an EXACT row that met an infinity or NaN comes from: its two parts
+// make NaN of 0 * inf and inf - inf, also by a later query's key in the same tile, where p * inf is
+// infinite and a masked key counts for nothing. Two walks, so that no infinite sum is ever rescaled.
+// (Not a fast path. Ordinary rows only pay for the test: 301 tokens at 211, 24 heads of 96, 13.5 -> 13.6 us;
+// a test of every element instead of their sum, 13.8.)
+template <int HD>
+__device__ __forceinline__ void plain_row(const float* __restrict__ qr, const _Float16* __restrict__ Kg,
+                                          const _Float16* __restrict__ Vg, size_t kv_dim, size_t n_keys, uint32_t hd,
+                                          float qscale, float* __restrict__ o) {
+    const uint32_t lane = threadIdx.x & 63;
+    auto score = [&](size_t key) {
+        const half8* kr = reinterpret_cast<const half8*>(Kg + min(key, n_keys - 1) * kv_dim);
+        float s = 0.f;
+        for (uint32_t c = 0; c < hd; c += 8) {
+            const half8 k8 = kr[c / 8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) s = fmaf(qr[c + e], float(k8[e]), s);
+        }
+        return key < n_keys ? s * qscale : -__builtin_inff();
+    };
+    float m = -__builtin_inff(), l = 0.f, acc[HD / 64] = {};
+    for (size_t k0 = 0; k0 < n_keys; k0 += 64) m = fmaxf(m, score(k0 + lane));
+    for (int s = 1; s < 64; s <<= 1) m = fmaxf(m, __shfl_xor(m, s));
+    for (size_t k0 = 0; k0 < n_keys; k0 += 64) {
+        const float p = k0 + lane < n_keys ? fast_exp2(score(k0 + lane) - m) : 0.f;
+        l += p;
+        for (uint32_t j = 0; j < min(size_t(64), n_keys - k0); j++) {
+            const float pj = __shfl(p, int(j));
+#pragma unroll
+            for (int d = 0; d < HD / 64; d++)
+                if (lane + 64 * d < hd) acc[d] = fmaf(pj, float(Vg[(k0 + j) * kv_dim + lane + 64 * d]), acc[d]);
+        }
+    }
+    for (int s = 1; s < 64; s <<= 1) l += __shfl_xor(l, s);
+#pragma unroll
+    for (int d = 0; d < HD / 64; d++)
+        if (lane + 64 * d < hd) o[lane + 64 * d] = acc[d] / l;
+}
+
 // EXACT: head sizes without a kernel of their own (hd < HD, a multiple of 8), one head per unit,
 // never split: the dims past hd are zero in LDS and not stored, and q and the probabilities enter
 // the MFMAs as two f16 parts each (together ~22 bits; K and V are f16 as stored), so that the scores
@@ -613,7 +653,20 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
     const uint32_t row = q0 + li;
     const bool live = row < n_tok;
     if (n_splits == 1) {  // the whole key range: write the output
-        if (!owner || !live) return;
+        if (!owner || (!EXACT && !live)) return;
+        bool plain = false;  // EXACT: this query met an infinity or NaN
+        uint32_t plain_rows = 0;
+        if constexpr (EXACT) {
+            float4v x = O[0][0];
+#pragma unroll
+            for (int d = 1; d < ND; d++) x += O[0][d];
+            // (tested by the exponent: -fno-honor-nans takes a float test for NaN out)
+            uint32_t bits = __float_as_uint((x[0] + x[1]) + (x[2] + x[3]));
+            asm("" : "+v"(bits));
+            const uint64_t met = __builtin_amdgcn_ballot_w64(live && (bits & 0x7fffffffu) >= 0x7f800000u);
+            plain_rows = uint32_t(met | met >> 16 | met >> 32 | met >> 48) & 0xffff;
+            plain = plain_rows >> li & 1;
+        }
         // Write-through (sc1) stores: the output leaves no dirty lines in the L2 for the
         // end-of-dispatch write-back (measured: C2 11.75 -> 11.19 us, C4 39.8 -> 38.5; a
         // nontemporal store gained less).
@@ -627,10 +680,16 @@ void attn_prefill_kernel(const float* __restrict__ q, const _Float16* __restrict
             const int off = int(4 * ((row - qblk0) * q_stride + head * hd + 4 * g));
 #pragma unroll
             for (int d = 0; d < ND; d++)
-                if (!EXACT || uint32_t(16 * d + 4 * g) < hd)
+                if (!EXACT || (live && !plain && uint32_t(16 * d + 4 * g) < hd))
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, O[h][d] * inv), ors, off + 64 * d,
                                                            0, kScDevice);
         }
+        if constexpr (EXACT)
+            for (; plain_rows != 0; plain_rows &= plain_rows - 1) {
+                const size_t r = q0 + uint32_t(__builtin_ctz(plain_rows));
+                plain_row<HD>(q + r * q_stride + size_t(kvh) * hd, Kg, Vg, kv_dim, size_t(pos) + r + 1, hd, qscale,
+                              out + r * q_stride + size_t(kvh) * hd);
+            }
         return;
     }
 

@@ -147,3 +147,44 @@ def test_any_finite_query(dev, hd, size):
     want = p / p.sum(1, keepdims=True) @ v.astype(np.float64)
     got = out.cpu().numpy()
     assert np.all(np.isfinite(got)) and np.linalg.norm(got - want) <= 2e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("hd", [8, 40, 96, 136, 200])
+@pytest.mark.parametrize("where", ["v", "k", "q"])
+def test_infinities(dev, hd, where):
+    """A value that became infinite (the f16 cache has no more above 65504) reaches what it is a part
+    of and nothing else: an infinite V element its dimension of the queries that see its key, a key
+    whose score is -inf no output, a query with a NaN itself. Every other element keeps the bar of
+    ordinary scores, also of queries before the key and of the same query's other dimensions."""
+    import torch
+    import ingot_attn as ia
+
+    nh, nkv, pos, n = 4, 2, 300, 150
+    L, kvd = pos + n, nkv * hd
+    rng = np.random.default_rng(hd)
+    q = rng.standard_normal((n, nh * hd)).astype(np.float32)
+    k = rng.standard_normal((L, kvd)).astype(np.float16)
+    v = rng.standard_normal((L, kvd)).astype(np.float16)
+    if where == "v":  # (KV head 0; of one sign in dimensions 0 and hd - 1, of both from key 400 on in 5)
+        v[pos + 40, 0], v[pos + 77, hd - 1], v[pos + 20, 5], v[pos + 100, 5] = np.inf, -np.inf, np.inf, -np.inf
+    elif where == "k":
+        q[:, :2 * hd:hd] = 1 + np.abs(q[:, :2 * hd:hd])  # (the heads of KV head 0)
+        k[33, 0], k[pos + 55, 0] = -np.inf, -np.inf
+    else:
+        q[70, hd + 3] = np.nan
+    t = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+    out = torch.zeros(n, nh * hd, device=dev)
+    ia.attn_prefill(t(q), t(k), t(v), out, ia.prefill_desc(nh, nkv, hd, pos, n))
+    got = out.cpu().numpy()
+    for h in range(nh):
+        c, kc = slice(h * hd, (h + 1) * hd), slice(h // 2 * hd, (h // 2 + 1) * hd)
+        with np.errstate(invalid="ignore"):
+            s = q[:, c].astype(np.float64) @ k[:, kc].astype(np.float64).T / np.sqrt(hd)
+            s[np.arange(L)[None, :] > pos + np.arange(n)[:, None]] = -np.inf
+            p = np.exp(s - s.max(1, keepdims=True))
+            vis = np.arange(L)[None, :, None] <= (pos + np.arange(n))[:, None, None]
+            want = np.where(vis, p[:, :, None] * v[None, :, kc].astype(np.float64), 0).sum(1) / p.sum(1, keepdims=True)
+        fin, g = np.isfinite(want), got[:, c]
+        assert np.array_equal(fin, np.isfinite(g)) and np.array_equal(want[~fin], g[~fin], equal_nan=True), h
+        assert np.linalg.norm(g[fin] - want[fin]) <= 2e-6 * np.linalg.norm(want[fin]), h
+        assert fin.mean() > 0.7 and fin.all() == (where == "k" or h > 1 or (where == "q" and h == 0)), h
