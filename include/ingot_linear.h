@@ -116,8 +116,9 @@ typedef struct IngotProjDesc {
  * INGOT_PROJ_X (else INGOT_ATTN_EUNSUPPORTED). With INGOT_PROJ_STORE or INGOT_PROJ_ACCUMULATE
  * each out[m] equals that of ingot_linear (n_tok, n_splits = 1) on matrix m, bit for bit. It
  * replaces the q/k/v encode_linear calls of a chunk (src/metal_backend.mm:440-442): the three
- * matrices' row tiles together fill the GPU better than each alone. (Matrices of up to 4096 rows
- * and of more in one call take one launch each kind.) With
+ * matrices' row tiles together fill the GPU better than each alone. (Matrices whose rows are summed
+ * in different numbers of k groups, which follow from type, n_in, n_out and n_tok, are launched
+ * apart; so are pieces of rows beyond 32-bit offsets.) With
  * INGOT_PROJ_SILU_GATE (two matrices of equal n_out) out[0] = silu(W[0]·x) * (W[1]·x) per
  * element, equal bit for bit to ingot_linear on each matrix (n_splits = 1) followed by
  * ingot_silu_mul; it replaces the gate and up encode_linear calls and encode_silu_mul of a chunk

@@ -16,7 +16,7 @@
 // What bounds it: a few tokens, the latency of the chain launch - first loads - walk - tail (13
 // tokens, 5120 x 3072 Q8_0: 57.7 us on one-k-group tiles of 256 rows, 18.6 here); a full chunk, the
 // x stream and the dequantization that the MFMAs wait for (512 tokens, gate/up of 3072 -> 2 x 8192
-// Q8_0: 124.6 -> 77 us, Q4_0 80.3 -> 65: 790 TFLOP/s, matrix cores busy 34% of the cycles); F16 and
+// Q8_0: 124.6 -> 77 us, Q4_0 80.3 -> 65: 790 TFLOP/s, matrix cores busy 35% of the counted cycles); F16 and
 // BF16 rows, HBM: with weights that no cache holds a square of 3072 at 512 tokens takes 32.6 us, from the
 // cache 25.5 (the kernel before this one 27.5 and 26.2; why it lost less is not known: two or three stages
 // of W or x more on their way gave 0.94 to 1.03x, x stages twice as long 0.84 to 1.03x). Measured
