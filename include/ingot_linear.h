@@ -69,8 +69,9 @@ size_t ingot_linear_workspace_size(const IngotLinearDesc* d);
  *              at all.
  * Deterministic: the split partials are summed in a fixed order, so equal inputs and equal
  * workspace sizes give bit-identical results; calls with and without a split differ by f32
- * rounding only. Not thread-safe per workspace (calls sharing one must be ordered on a
- * stream). */
+ * rounding only, as do rows of x at different places of a call (n_splits != 1 with a workspace:
+ * the order of a sum may depend on the token's tile). Not thread-safe per workspace (calls
+ * sharing one must be ordered on a stream). */
 int ingot_linear(const void* w, const float* x, float* out, void* workspace, size_t workspace_bytes,
                  const IngotLinearDesc* d, void* stream);
 

@@ -867,7 +867,8 @@ int launch_t(const uint8_t* W, const float* x, float* out, uint32_t n_in, uint32
         return launch_matvec_t<T>(a, 1, kProNone, accumulate ? kEpiAccumulate : kEpiStore, stream);
     }
     TileCall c{{W}, {out}, {n_out}, 1, x, n_in, n_tok, accumulate != 0, false,
-               linear_shape(T, n_in, n_out, n_tok, workspace ? n_splits : 1, workspace_bytes), workspace, stream};
+               linear_shape(T, n_in, n_out, n_tok, workspace ? n_splits : 1, workspace_bytes), workspace, stream,
+               workspace && n_splits != 1};
     return launch_tile<T>(c);
 }
 

@@ -30,6 +30,7 @@ struct TileCall {
     TileShape shape;
     void* workspace;  // counters, then partial tiles (shape.splits > 1)
     hipStream_t stream;
+    bool spread = false;  // the order of the sums is free (see tile_spread)
     uint32_t row0 = 0, rows = ~0u;  // the rows of each matrix to compute (out keeps its n_out columns)
 };
 
@@ -56,6 +57,16 @@ constexpr size_t tile_lds(uint32_t ntb, uint32_t kg, size_t w) {
 }
 constexpr size_t tile_bytes(const TileShape& s) { return size_t(tile_rows(s.kg)) * s.ntb * 32 * 4; }
 
+// Do the token tiles of a call start their walks of n_in apart? It pays where what one tile has read stays
+// in the XCD's 4 MB of L2 until the last has (w: bytes of the rows, an eighth on each XCD; x: bytes of x),
+// measured on two k groups (with weights from HBM, 2 to 1024 tokens, 0.90 to 1.20x of in step): F16 and BF16
+// 1.047x in the mean up to w = 20 MB and x = 9 MB (3072 x 3072: 256 tokens 24.0 -> 21.4 us, 512 34.4 ->
+// 28.7; the worst, 1024 x 4096 at 700, 18.2 -> 20.3), 0.91 to 0.96x with w = 33 MB or with w = 17 MB and x from 9.4 MB on; Q8_0, Q4_0 and Q4_1 1.02x,
+// Q6_K 1.00x. On one k group 256 rows share a walk and lose more than they gain from 2 MB on (0.98x,
+// 0.92x, 0.89x at 2, 4 and 7 MB an XCD); calls on four have few token tiles.
+inline bool tile_spread(const TileShape& s, uint64_t w, uint64_t x) {
+    return s.kg == 2 && w <= 20000000 && x <= 9000000;
+}
 // First of part i's share where n things are spread evenly over `parts`, the first n % parts parts one
 // longer: the token blocks of a token tile, the k units of a split. (i * n / parts would pass 32 bits
 // from 2.1 million tokens of one-block tiles, 4.2 million of four-block tiles on.)

@@ -16,10 +16,10 @@
 // What bounds it: a few tokens, the latency of the chain launch - first loads - walk - tail (13
 // tokens, 5120 x 3072 Q8_0: 57.7 us on one-k-group tiles of 256 rows, 18.6 here); a full chunk, the
 // x stream and the dequantization that the MFMAs wait for (512 tokens, gate/up of 3072 -> 2 x 8192
-// Q8_0: 124.6 -> 77 us, Q4_0 80.3 -> 65: 790 TFLOP/s, matrix cores busy 35% of the counted cycles); F16 and
-// BF16 rows, HBM: with weights that no cache holds a square of 3072 at 512 tokens takes 32.6 us, from the
-// cache 25.5 (the kernel before this one 27.5 and 26.2; why it lost less is not known: two or three stages
-// of W or x more on their way gave 0.94 to 1.03x, x stages twice as long 0.84 to 1.03x). Measured
+// Q8_0: 124.6 -> 77 us, Q4_0 80.3 -> 65: 790 TFLOP/s, matrix cores busy 35% of the counted cycles).
+// Token tiles that walk the same rows in step all wait for HBM at every stage: a square of 3072 in F16
+// with weights that no cache holds took 32.4 us at 512 tokens, from the cache 25.5 (the kernel before
+// this one 27.5); with their walks spread over the rows (tile_spread) 27.2. Measured
 // on the way there, 512 tokens of Q4_0 gate/up: weights read by each lane straight from memory
 // made the L1 fetch every line 5 times over (7.5 M line reads a launch, 5.3 M with whole rows
 // through LDS); a branch around the dequantization of a ragged end kept the compiler from
@@ -164,7 +164,7 @@ struct TileArgs {
     uint32_t tile_end[2];  // row tiles of matrix m: [tile_end[m-1], tile_end[m])
     const float* x;
     uint32_t n_in, n_tok, row_bytes, accumulate;
-    uint32_t tiles_n, tiles_m, splits, units, per_xcd;
+    uint32_t tiles_n, tiles_m, splits, units, per_xcd, spread;
     float* part;
     unsigned int* counters;
 };
@@ -231,10 +231,22 @@ void linear_tile_kernel(const TileArgs a) {
         wl[i] = (r * WS::pitch + 16 * o) | o;  // (o < 16: the chunk's place rides along)
     }
     const uint32_t live = min(klen, a.n_in > kg0 ? a.n_in - kg0 : 0u) / 32;  // columns of the share within n_in
-    auto load_w = [&](uint32_t w) {  // W stage w of the share
+    // Where a.spread, the token tiles that share these rows start their walks evenly apart and wrap: each
+    // brings a part of the rows into the L2 for all of them (in step they would all wait for HBM at every stage).
+    constexpr uint32_t M = QS > U ? QS : U;  // steps of whole W and x stages
+    static_assert(M % QS == 0 && M % U == 0, "whole stages");
+    uint32_t first = 0;
+    if constexpr (KG == 2 && !PAIR)
+        if (a.spread && !ragged && steps % M == 0) first = tt * (steps / M) / a.tiles_m * M;
+    auto w_stage = [&](uint32_t w) {
+        const uint32_t at = w + first / QS;
+        return first != 0 && at >= steps / QS ? at - steps / QS : at;
+    };
+    auto load_w = [&](uint32_t w) {  // W stage w of the walk
+        const uint32_t at = w_stage(w) * WSB;
 #pragma unroll
         for (uint32_t i = 0; i < NCH; i++) {
-            uint32_t off = ((wa[i] + w * WSB) & ~15u) + 16 * (wl[i] & 15);
+            uint32_t off = ((wa[i] + at) & ~15u) + 16 * (wl[i] & 15);
             if constexpr (Fmt<T>::blk == 1)  // (a chunk past the end loads zeros; a block's scale is cleared in col_frag)
                 if (w * WS::WK + 16 / Fmt<T>::bytes * (wl[i] & 15) >= 32 * live) off = kOob;
             wr[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, int(off), 0, 0));
@@ -249,7 +261,7 @@ void linear_tile_kernel(const TileArgs a) {
     uint32_t wraw[2][Col<T>::ndw], woff[2];
     auto read_w = [&](int s, uint32_t j) {
         const uint32_t i = 2 * (j % QS) + h;
-        woff[s] = ((roff + j / QS * WSB) & 15) + col_offset<T>(i);
+        woff[s] = ((roff + w_stage(j / QS) * WSB) & 15) + col_offset<T>(i);
         col_read<T>(wsm + n * WS::pitch, woff[s], i, wraw[s]);
     };
     auto frag_of = [&](int s, uint32_t j, int e) {
@@ -273,7 +285,8 @@ void linear_tile_kernel(const TileArgs a) {
 #pragma unroll
     for (uint32_t i = 0; i < NX; i++) xo[i] = tr + RPP * i < toks ? 4 * ((tr + RPP * i) * a.n_in + xk) : kOob;
     auto load_x = [&](uint32_t j, uint32_t i0, uint32_t i1) {  // pieces i0..i1-1 of stage j
-        const uint32_t k = 64 * U * min(j, nst - 1);  // (past the share: its last stage again)
+        const uint32_t at = min(j, nst - 1) + first / U;  // (past the walk: its last stage again)
+        const uint32_t k = 64 * U * (at >= nst ? at - nst : at);
         const bool cut = ragged && (xi + k >= klen || xk + k >= a.n_in);
 #pragma unroll
         for (uint32_t i = 0; i < NX; i++)
@@ -569,6 +582,7 @@ int launch_tile(const TileCall& c) {
     a.tiles_m = ((c.n_tok + 31) / 32 + ntb - 1) / ntb;
     a.units = tile_units(T, c.n_in, kg);
     a.splits = c.shape.splits;
+    a.spread = c.spread && tile_spread(c.shape, uint64_t(c.n_out[0]) * row_bytes, c.n_tok * x_bytes);
     if (a.splits == 0 || a.splits > std::min(a.units, 8u)) return -1;
     const uint64_t total = uint64_t(a.tiles_n) * a.tiles_m * a.splits, per_xcd = (total + 7) / 8;
     if (per_xcd * 8 > 0x7fffffffu) return -1;

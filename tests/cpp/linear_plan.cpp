@@ -20,3 +20,8 @@ extern "C" void plan_shape(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_
 extern "C" void plan_pair(uint32_t type, uint32_t n_in, uint32_t n_out, uint32_t n_tok, uint32_t* out) {
     put(ingot::unsplit_shape(type, n_in, 2 * n_out, n_tok, ingot::unsplit_k_groups(type, n_in, n_out, n_tok)), out);
 }
+
+// Do the token tiles of an ingot_linear call of that shape start apart?
+extern "C" bool plan_spread(uint32_t kg, uint64_t weight_bytes, uint64_t x_bytes) {
+    return ingot::tile_spread(ingot::TileShape{1, kg, 1}, weight_bytes, x_bytes);
+}

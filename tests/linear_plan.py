@@ -59,3 +59,20 @@ def smallest(t):
             one.setdefault((b, kg, splits > 1), (n_in, n_out, n_tok, req))
         two.setdefault(pair(t, n_in, n_out, n_tok)[:2], (n_in, n_out, n_tok))
     return one, two
+
+
+@functools.lru_cache(maxsize=None)
+def spread(t):
+    """{(token blocks, split?, more than two token tiles?): (n_in, n_out, n_tok, n_splits)}: the call of
+    least work whose token tiles start apart (whole stages of weights: 256 elements of every k group)."""
+    per = {"F32": 4, "F16": 2, "BF16": 2, "Q8_0": 34 / 32, "Q4_0": 18 / 32, "Q4_1": 20 / 32, "Q6_K": 210 / 256}[t]
+    out = {}
+    sizes = [(i, o, n) for i in (1024, 1536, 2560, 3072, 4096) for o in (130, 257, 514, 1025, 2050, 3073)
+             for n in (65, 97, 129, 161, 200, 257, 321, 390, 450, 513, 600, 700)]
+    for n_in, n_out, n_tok in sorted(sizes, key=lambda s: s[0] * s[1] * s[2]):
+        for req in (0, 2, 3, 4):
+            b, kg, splits = linear(t, n_in, n_out, n_tok, req)
+            tiles = -(-(-(-n_tok // 32)) // b)
+            if tiles > 1 and n_in % (512 * splits) == 0 and lib().plan_spread(kg, ctypes.c_uint64(int(n_in * n_out * per)), ctypes.c_uint64(4 * n_in * n_tok)):
+                out.setdefault((b, splits > 1, tiles > 2), (n_in, n_out, n_tok, req))
+    return out

@@ -65,6 +65,15 @@ def test_every_kernel(dev, oracle_mod, t):
 
 
 @pytest.mark.parametrize("t", lp.TYPES)
+def test_walks_spread_over_the_rows(dev, oracle_mod, t):
+    """Token tiles that start their walks of n_in at different stages and wrap: two and more of them,
+    split and not, every tile height."""
+    assert len(lp.spread(t)) >= 4 and len({k[0] for k in lp.spread(t)}) >= 2
+    for key, case in lp.spread(t).items():
+        _linear(dev, oracle_mod, t, *case, (key, case))
+
+
+@pytest.mark.parametrize("t", lp.TYPES)
 def test_every_pair_kernel(dev, oracle_mod, t):
     """silu(gate) * up of each tile: equal bit for bit to the two products (n_splits = 1) and
     ingot_silu_mul, and near the oracle's sums (silu' <= 1.1: the bar on the sums, times |up| and |gate|)."""
