@@ -16,7 +16,7 @@
 // What bounds it: a few tokens, the latency of the chain launch - first loads - walk - tail (13
 // tokens, 5120 x 3072 Q8_0: 57.7 us on one-k-group tiles of 256 rows, 18.6 here); a full chunk, the
 // x stream and the dequantization that the MFMAs wait for (512 tokens, gate/up of 3072 -> 2 x 8192
-// Q8_0: 124.6 -> 77 us, Q4_0 80.3 -> 65: 790 TFLOP/s, matrix cores busy 35% of the counted cycles).
+// Q8_0: 124.6 -> 77 us, Q4_0 80.3 -> 65: 790 TFLOP/s, matrix cores busy 34% of the counted cycles).
 // Token tiles that walk the same rows in step all wait for HBM at every stage: a square of 3072 in F16
 // with weights that no cache holds took 32.4 us at 512 tokens, from the cache 25.5 (the kernel before
 // this one 27.5); with their walks spread over the rows (tile_spread) 27.2. Measured
@@ -24,7 +24,7 @@
 // made the L1 fetch every line 5 times over (7.5 M line reads a launch, 5.3 M with whole rows
 // through LDS); a branch around the dequantization of a ragged end kept the compiler from
 // interleaving MFMAs with it (67 M wave-cycles, 52 M without); starting the token tiles at
-// different stages, as the L2 channels would like it, changed nothing.
+// different stages changed nothing there (rows of that size do not stay in the L2).
 #include <algorithm>
 #include <type_traits>
 
